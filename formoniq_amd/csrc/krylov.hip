@@ -1301,10 +1301,11 @@ static void minres_iteration(Enq& q, MinresWork<T>& w, const int64_t* rp, const 
 }
 
 // Iterations per segment. A segment ends with a host read of the MINRES
-// scalars, and work that other contexts queue meanwhile waits behind the
-// segments already on the device (one request's set-up syncs wait for another
-// request's segment), so a segment holds about 16 ms of estimated work: bytes
-// per iteration at 4 TB/s plus 4 us per kernel; even, 2..graph_iters.
+// scalars, about 15 us with the relaunch; iterations past the stopping one run
+// as launches that return at once, 1.3 us each, and the graph's build grows
+// with its nodes. A segment holds about 0.5 ms of estimated work: bytes per
+// iteration at 4 TB/s plus 2.5 us per kernel; even, 2..graph_iters. (Short
+// segments also keep other contexts' set-up from queueing behind a solve.)
 template <class T>
 static int segment_iters(const MinresWork<T>& w, const feec_solve_opts& o) {
   const double vb = sizeof(T), N = (double)(w.n + w.nh);
@@ -1322,8 +1323,8 @@ static int segment_iters(const MinresWork<T>& w, const feec_solve_opts& o) {
     bytes += (double)hx_bytes_per_apply(*w.hx) * (std::is_same_v<T, float> || w.hx_fp32 ? 1.0 : 1.6);
     launches += hx_launches_per_apply(*w.hx);
   }
-  const double t = bytes / 4e12 + launches * 4e-6;
-  const int seg = (int)std::min(1e6, 0.016 / t);
+  const double t = bytes / 4e12 + launches * 2.5e-6;
+  const int seg = (int)std::min(1e6, 0.5e-3 / t);
   const int cap = std::max(2, o.graph_iters - (o.graph_iters & 1));
   return std::clamp(seg - (seg & 1), 2, cap);
 }

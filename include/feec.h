@@ -102,8 +102,9 @@ typedef struct feec_solve_opts {
   double inner_rtol;     /* mixed: FP32 inner MINRES tolerance (default 1e-4) */
   int32_t use_graph;     /* capture Krylov iterations in a hipGraph (default 1) */
   int32_t graph_iters;   /* most iterations per graph segment, even (default 32); a segment is
-                            cut to about 16 ms of estimated device work, so that other
-                            contexts' work does not queue long behind it */
+                            cut to about 0.5 ms of estimated device work, so that few launches
+                            run past the stopping iteration and other contexts' work does not
+                            queue long behind it */
   int32_t cheb_degree;   /* degree of the Chebyshev-Jacobi polynomial applied to each
                             hdif_gram block of the preconditioner; 0 = Jacobi only; -1 = by
                             mesh resolution r = N_0^(1/d): 8 sqrt(r) in multiples of 8 within
