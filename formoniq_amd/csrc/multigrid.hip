@@ -48,9 +48,8 @@
 // is not an unknown. Vertices that are not unknowns (the boundary of the
 // relative complex, their coarse counterparts) are "dead": zero rows and
 // columns and a zero smoother entry, so they stay zero through the cycle.
-// Slot vectors are interleaved, x[i * nv + slot], and the cycle's kernels run
-// one thread per (vertex, slot), so every vector access of a wavefront is
-// contiguous and no column index is read. The prolongation and restriction
+// Slot vectors lie one after the other, x[slot * nb + i], so every vector
+// access of a wavefront is contiguous and no column index is read. The prolongation and restriction
 // are computed from grid coordinates, without matrices.
 //
 // Precision. The FP64 path runs every piece in FP64; the mixed paths in FP32
@@ -141,7 +140,7 @@ __global__ void __launch_bounds__(TPB) k_st_scale(const TP* __restrict__ dinv, c
   if (skip(S)) return;
   const unsigned t = xcd_block() * blockDim.x + threadIdx.x;
   if (t >= nb * nv) return;
-  x[t] = dinv[t / nv] * r[t];
+  x[t] = dinv[t % nb] * r[t];
 }
 
 // The sweep family, one thread per (vertex, slot). The operator is
@@ -154,9 +153,9 @@ __global__ void __launch_bounds__(TPB) k_st_scale(const TP* __restrict__ dinv, c
 // FINE marks the finest level's launches, which stream the operator from HBM,
 // as their own instantiation (the coarse levels are cache-resident).
 template <class TP, int MODE>
-__device__ __forceinline__ TP st_iterate(int j, unsigned nv, unsigned v, const TP* __restrict__ x,
-                                         const TP* __restrict__ dinv, const TP* __restrict__ r) {
-  return MODE == 2 ? dinv[j] * r[(unsigned)j * nv + v] : x[(unsigned)j * nv + v];
+__device__ __forceinline__ TP st_iterate(int j, const TP* __restrict__ x, const TP* __restrict__ dinv,
+                                         const TP* __restrict__ r) {
+  return MODE == 2 ? dinv[j] * r[j] : x[j];
 }
 
 template <class TP, int D, int MODE, bool FINE>
@@ -168,9 +167,11 @@ __global__ void __launch_bounds__(TPB) k_st_sweep(const TP* __restrict__ A, cons
   const unsigned t = xcd_block() * blockDim.x + threadIdx.x;
   const unsigned nb = (unsigned)b.nb;
   if (t >= nb * nv) return;
-  const unsigned i = t / nv;
-  const unsigned v = t - i * nv;
-  const TP xi = st_iterate<TP, MODE>((int)i, nv, v, x, dinv, r);
+  const unsigned base = t / nb * nb;  // the slot's vectors
+  const unsigned i = t - base;
+  r += base;
+  x += base;
+  const TP xi = st_iterate<TP, MODE>((int)i, x, dinv, r);
   TP acc = A[i] * xi;
 #pragma unroll
   for (int m = 1; m <= H; ++m) {
@@ -182,11 +183,11 @@ __global__ void __launch_bounds__(TPB) k_st_sweep(const TP* __restrict__ A, cons
     const TP am = jm >= 0 ? A[(size_t)m * nb + jm] : TP(0);
     jp = jp < (int)nb ? jp : (int)i;
     jm = jm >= 0 ? jm : (int)i;
-    acc += ap * st_iterate<TP, MODE>(jp, nv, v, x, dinv, r);
-    acc += am * st_iterate<TP, MODE>(jm, nv, v, x, dinv, r);
+    acc += ap * st_iterate<TP, MODE>(jp, x, dinv, r);
+    acc += am * st_iterate<TP, MODE>(jm, x, dinv, r);
   }
   const TP d = dinv[i];
-  const TP res = r[t] - acc;
+  const TP res = r[i] - acc;
   out[t] = MODE == 1 ? (d != TP(0) ? res : TP(0)) : xi + d * res;
 }
 
@@ -200,8 +201,8 @@ __global__ void __launch_bounds__(TPB) k_st_restrict(const TP* __restrict__ ef, 
   if (skip(S)) return;
   const unsigned t = xcd_block() * blockDim.x + threadIdx.x;
   if (t >= (unsigned)cb.nb * nv) return;
-  const unsigned w = t / nv;
-  const unsigned v = t - w * nv;
+  const unsigned v = t / (unsigned)cb.nb;
+  const unsigned w = t - v * (unsigned)cb.nb;
   if (!live_c[w]) {
     rc[t] = TP(0);
     return;
@@ -228,7 +229,7 @@ __global__ void __launch_bounds__(TPB) k_st_restrict(const TP* __restrict__ ef, 
       in = in && c >= 0 && c <= fb.g;
       k += c * fb.st[a];
     }
-    if (in) acc += (s == 0 ? TP(1) : TP(0.5)) * ef[(unsigned)k * nv + v];
+    if (in) acc += (s == 0 ? TP(1) : TP(0.5)) * ef[v * (unsigned)fb.nb + (unsigned)k];
   }
   rc[t] = acc;
 }
@@ -241,9 +242,10 @@ __global__ void __launch_bounds__(TPB) k_st_prolong(const TP* __restrict__ xc, T
   if (skip(S)) return;
   const unsigned t = xcd_block() * blockDim.x + threadIdx.x;
   if (t >= (unsigned)fb.nb * nv) return;
-  const unsigned k = t / nv;
-  const unsigned v = t - k * nv;
+  const unsigned v = t / (unsigned)fb.nb;
+  const unsigned k = t - v * (unsigned)fb.nb;
   if (dinv_f[k] == TP(0)) return;
+  xc += v * (unsigned)cb.nb;
   unsigned r = k;
   int lo = 0, hi = 0;
   bool odd = false;
@@ -255,9 +257,7 @@ __global__ void __launch_bounds__(TPB) k_st_prolong(const TP* __restrict__ xc, T
     hi += ((c >> 1) + (c & 1)) * cb.st[a];
     odd = odd || (c & 1);
   }
-  const TP add = odd ? TP(0.5) * (xc[(unsigned)lo * nv + v] + xc[(unsigned)hi * nv + v])
-                     : xc[(unsigned)lo * nv + v];
-  xf[t] += add;
+  xf[t] += odd ? TP(0.5) * (xc[lo] + xc[hi]) : xc[lo];
 }
 
 // x = C r on the coarsest box, C dense (nb x nb, row-major, zero on dead
@@ -275,7 +275,7 @@ __global__ void __launch_bounds__(TPB) k_st_dense(const TP* __restrict__ C, cons
     const TP c = C[(size_t)i * nb + j];
 #pragma unroll
     for (int v = 0; v < MAXNV; ++v)
-      if (v < nv) acc[v] += c * r[j * nv + v];
+      if (v < nv) acc[v] += c * r[v * nb + j];
   }
 #pragma unroll
   for (int v = 0; v < MAXNV; ++v) {
@@ -289,7 +289,567 @@ __global__ void __launch_bounds__(TPB) k_st_dense(const TP* __restrict__ C, cons
   if (threadIdx.x < (unsigned)nv) {
     TP t = TP(0);
     for (int w = 0; w < TPB / 64; ++w) t += sh[w][threadIdx.x];
-    x[i * nv + threadIdx.x] = t;
+    x[threadIdx.x * nb + i] = t;
+  }
+}
+
+template <int D, int P>
+__host__ __device__ constexpr int tail_stride(int a) {
+  int s = 1;
+  for (int i = 0; i < a; ++i) s *= P;
+  return s;
+}
+// the offset of the +delta neighbour m in a cube of pitch P
+template <int D, int P>
+__host__ __device__ constexpr int tail_offset(int m) {
+  int o = 0;
+  for (int a = 0; a < D; ++a)
+    if (m & (1 << a)) o += tail_stride<D, P>(a);
+  return o;
+}
+
+// ---------------------------------------------------------------------------
+// a level of the V-cycle in two launches (two sweeps, d <= 3)
+// ---------------------------------------------------------------------------
+// Down: x = dinv r, a sweep, the residual and its restriction; up: the
+// correction and two sweeps. A workgroup takes one slot of a tile and
+// recomputes the halo, its vectors in LDS, its vertices' operator rows in
+// registers: one launch in place of three. A lone workgroup takes about 6 us
+// (4 of them its loads), so this pays where all of them run at once, on levels
+// whose separate kernels are bound by the launch: 3D 21^3, 5 slots: 16 us
+// against 26 for the six, 17^3: 15 against 22; with more workgroups than the
+// chip holds the halo's work costs more than the launches (65^3: 75 against
+// 50, 28^3 with 10 slots: 31 against 28).
+constexpr int TILE_TPB = 512;
+template <int D>
+constexpr int kTile = D == 1 ? 128 : D == 2 ? 16 : 4;  // coarse vertices an axis of a tile
+__host__ __device__ constexpr int cpow(int b, int e) { return e == 0 ? 1 : b * cpow(b, e - 1); }
+
+// The operator's row at box vertex i. A position off the box holds a zero of
+// the vector in LDS, so an element there (in: false) only needs d = 0 and the
+// coefficients towards it may be any; the loads are unconditional, each from a
+// uniform address plus the vertex's own offset.
+template <class TP, int D>
+struct TileRow {
+  TP a0, p[(1 << D) - 1], m[(1 << D) - 1], d;
+};
+template <class TP, int D>
+__device__ __forceinline__ void tile_row(TileRow<TP, D>& w, const TP* __restrict__ A, const TP* __restrict__ dinv,
+                                         const Box& b, unsigned i, bool in) {
+  constexpr int H = (1 << D) - 1;
+  w.a0 = A[i];
+#pragma unroll
+  for (int m = 1; m <= H; ++m) {
+    const TP* Am = A + m * b.nb;
+    w.p[m - 1] = Am[i];
+    w.m[m - 1] = (Am - stencil_offset<D>(m, b.st))[i];
+  }
+  const TP d = dinv[i];
+  w.d = in ? d : TP(0);
+}
+// r - A x at LDS position q (pitch P)
+template <class TP, int D, int P>
+__device__ __forceinline__ TP tile_residual(const TileRow<TP, D>& w, TP r, const TP* q) {
+  constexpr int H = (1 << D) - 1;
+  TP acc = w.a0 * *q;
+#pragma unroll
+  for (int m = 1; m <= H; ++m) {
+    acc += w.p[m - 1] * q[tail_offset<D, P>(m)];
+    acc += w.m[m - 1] * q[-tail_offset<D, P>(m)];
+  }
+  return r - acc;
+}
+// the tile's origin (in tiles) from its number
+template <int D>
+__device__ __forceinline__ void tile_origin(unsigned t, int n, int (&o)[D]) {
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    o[a] = (int)(t % (unsigned)n);
+    t /= (unsigned)n;
+  }
+}
+// Element idx of a cube of E positions an axis, `off` inside a cube of pitch P:
+// its LDS position, its vertex (0 off the box), whether it lies in the box, and
+// whether it is at least `rim` away from the cube's faces.
+template <int D, int E, int P>
+__device__ __forceinline__ void tile_at(int idx, int off, const int (&org)[D], const Box& b, int& pos, unsigned& i,
+                                        bool& in, bool& inner, int rim) {
+  pos = 0;
+  int j = 0;
+  in = inner = true;
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    const int l = idx % E;
+    idx /= E;
+    const int f = org[a] + l;
+    pos += (l + off) * tail_stride<D, P>(a);
+    j += f * b.st[a];
+    in = in && (unsigned)f <= (unsigned)b.g;
+    inner = inner && l >= rim && l < E - rim;
+  }
+  i = in ? (unsigned)j : 0u;
+}
+
+template <class TP, int D>
+__global__ void __launch_bounds__(TILE_TPB) k_st_down(const TP* __restrict__ A, const TP* __restrict__ dinv,
+                                                      const TP* __restrict__ r, TP* __restrict__ x,
+                                                      TP* __restrict__ rc, const uint8_t* __restrict__ live_c,
+                                                      Box fb, Box cb, int tiles, const MinresS* S) {
+  constexpr int T = kTile<D>, P = 2 * T + 5, E = 2 * T + 3, N0 = cpow(P, D), N1 = cpow(E, D), H = (1 << D) - 1;
+  constexpr int K0 = (N0 + TILE_TPB - 1) / TILE_TPB, K1 = (N1 + TILE_TPB - 1) / TILE_TPB;
+  if (skip(S)) return;
+  __shared__ TP sr[N0], s0[N0], s1[N0];
+  const int tid = threadIdx.x;
+  r += (int64_t)blockIdx.y * fb.nb;  // this workgroup's slot
+  x += (int64_t)blockIdx.y * fb.nb;
+  rc += (int64_t)blockIdx.y * cb.nb;
+  int to[D], o0[D], o1[D];
+  tile_origin<D>(xcd_block(), tiles, to);
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    o0[a] = 2 * T * to[a] - 3;
+    o1[a] = 2 * T * to[a] - 2;
+  }
+  TP d0[K0], r0[K0];
+#pragma unroll
+  for (int k = 0; k < K0; ++k) {
+    int pos;
+    unsigned i;
+    bool in, inner;
+    tile_at<D, P, P>(tid + k * TILE_TPB, 0, o0, fb, pos, i, in, inner, 0);
+    r0[k] = r[i];
+    const TP d = dinv[i];
+    d0[k] = in ? d : TP(0);
+  }
+  TileRow<TP, D> w[K1];
+  unsigned i1[K1];
+  int pos1[K1];
+  bool own[K1], mid[K1];
+#pragma unroll
+  for (int k = 0; k < K1; ++k) {
+    const int idx = tid + k * TILE_TPB;
+    bool in;
+    tile_at<D, E, P>(idx, 1, o1, fb, pos1[k], i1[k], in, mid[k], 1);
+    mid[k] = mid[k] && idx < N1;
+    if (idx >= N1) pos1[k] = 0;
+    tile_row<TP, D>(w[k], A, dinv, fb, i1[k], in);
+    own[k] = in && idx < N1;  // the tile's own vertices: 2T an axis from 2T * tile on
+    int q = idx;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      const int l = q % E;
+      q /= E;
+      own[k] = own[k] && l >= 2 && l < 2 + 2 * T;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K0; ++k) {
+    const int idx = tid + k * TILE_TPB;
+    if (idx < N0) {
+      sr[idx] = r0[k];
+      s0[idx] = d0[k] * r0[k];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K1; ++k)
+    if (tid + k * TILE_TPB < N1) {
+      const TP* q = s0 + pos1[k];
+      const TP xn = *q + w[k].d * tile_residual<TP, D, P>(w[k], sr[pos1[k]], q);
+      s1[pos1[k]] = xn;
+      if (own[k]) x[i1[k]] = xn;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K1; ++k)
+    if (mid[k]) s0[pos1[k]] = w[k].d != TP(0) ? tile_residual<TP, D, P>(w[k], sr[pos1[k]], s1 + pos1[k]) : TP(0);
+  __syncthreads();
+  for (int idx = tid; idx < cpow(T, D); idx += TILE_TPB) {
+    int q = idx, j = 0;
+    const TP* e = s0;
+    bool in = true;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      const int l = q % T;
+      q /= T;
+      const int c = T * to[a] + l;
+      in = in && c <= cb.g;
+      j += c * cb.st[a];
+      e += (2 * l + 3) * tail_stride<D, P>(a);
+    }
+    if (in) {
+      TP acc = TP(0);
+#pragma unroll
+      for (int m = 1; m <= H; ++m) acc += e[tail_offset<D, P>(m)] + e[-tail_offset<D, P>(m)];
+      rc[(unsigned)j] = live_c[(unsigned)j] ? *e + TP(0.5) * acc : TP(0);
+    }
+  }
+}
+
+// out = two sweeps from x + P xc
+template <class TP, int D>
+__global__ void __launch_bounds__(TILE_TPB) k_st_up(const TP* __restrict__ A, const TP* __restrict__ dinv,
+                                                    const TP* __restrict__ r, const TP* __restrict__ x,
+                                                    const TP* __restrict__ xc, TP* __restrict__ out, Box fb,
+                                                    Box cb, int tiles, const MinresS* S) {
+  constexpr int T = kTile<D>, P = 2 * T + 4, E = 2 * T + 2, N0 = cpow(P, D), N1 = cpow(E, D);
+  constexpr int K0 = (N0 + TILE_TPB - 1) / TILE_TPB, K1 = (N1 + TILE_TPB - 1) / TILE_TPB;
+  if (skip(S)) return;
+  __shared__ TP s0[N0], s1[N0];
+  const int tid = threadIdx.x;
+  r += (int64_t)blockIdx.y * fb.nb;  // this workgroup's slot
+  x += (int64_t)blockIdx.y * fb.nb;
+  out += (int64_t)blockIdx.y * fb.nb;
+  xc += (int64_t)blockIdx.y * cb.nb;
+  int to[D], o0[D], o1[D];
+  tile_origin<D>(xcd_block(), tiles, to);
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    o0[a] = 2 * T * to[a] - 2;
+    o1[a] = 2 * T * to[a] - 1;
+  }
+  TP x0[K0], cl[K0], ch[K0], d0[K0];
+  bool in0[K0];
+#pragma unroll
+  for (int k = 0; k < K0; ++k) {
+    int pos;
+    unsigned i;
+    bool inner;
+    const int idx = tid + k * TILE_TPB;
+    tile_at<D, P, P>(idx, 0, o0, fb, pos, i, in0[k], inner, 0);
+    int q = idx, lo = 0, hi = 0;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      const int f = o0[a] + q % P;
+      q /= P;
+      lo += (f >> 1) * cb.st[a];
+      hi += ((f + 1) >> 1) * cb.st[a];
+    }
+    x0[k] = x[i];
+    d0[k] = dinv[i];
+    cl[k] = xc[in0[k] ? (unsigned)lo : 0u];
+    ch[k] = xc[in0[k] ? (unsigned)hi : 0u];
+  }
+  TileRow<TP, D> w[K1];
+  TP r1[K1];
+  unsigned i1[K1];
+  int pos1[K1];
+  bool mid[K1];
+#pragma unroll
+  for (int k = 0; k < K1; ++k) {
+    const int idx = tid + k * TILE_TPB;
+    bool in;
+    tile_at<D, E, P>(idx, 1, o1, fb, pos1[k], i1[k], in, mid[k], 1);
+    mid[k] = mid[k] && in && idx < N1;
+    if (idx >= N1) pos1[k] = 0;
+    tile_row<TP, D>(w[k], A, dinv, fb, i1[k], in);
+    r1[k] = r[i1[k]];
+  }
+#pragma unroll
+  for (int k = 0; k < K0; ++k)
+    if (tid + k * TILE_TPB < N0)  // a dead vertex takes no correction
+      s0[tid + k * TILE_TPB] = in0[k] ? x0[k] + (d0[k] != TP(0) ? TP(0.5) : TP(0)) * (cl[k] + ch[k]) : TP(0);
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K1; ++k)
+    if (tid + k * TILE_TPB < N1) {
+      const TP* q = s0 + pos1[k];
+      s1[pos1[k]] = *q + w[k].d * tile_residual<TP, D, P>(w[k], r1[k], q);
+    }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K1; ++k)
+    if (mid[k]) {
+      const TP* q = s1 + pos1[k];
+      out[i1[k]] = *q + w[k].d * tile_residual<TP, D, P>(w[k], r1[k], q);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// the coarse end of the V-cycle in one launch
+// ---------------------------------------------------------------------------
+// Levels t0 .. last of the cycle, one workgroup per slot, every phase ending at
+// a workgroup barrier instead of a launch: on these levels a kernel of the
+// sweep family moves a few hundred kilobytes and takes what a launch takes
+// (2-4 us). The slot's vectors lie in LDS; the first of the levels keeps its
+// operator and right-hand side in registers, K vertices a lane, the others keep
+// theirs in LDS, so that each phase costs its LDS reads and not a round trip
+// to the cache (with the operators read from cache in every phase the launch
+// took as long as the 13 it replaced).
+constexpr int TAIL_TPB = 1024;
+constexpr int TAIL_LDS = 160 * 1024;
+constexpr int TAIL_LEVELS = 8;
+// Vertices a lane of the first level: 2^(d+1) - 1 coefficients each, in the
+// 128 registers that 16 wavefronts a CU leave. The first level's vectors take
+// a fixed pitch in LDS (its cube root of lanes times vertices, plus two), so
+// that every neighbour is the vertex's position plus a constant, a read of the
+// instruction's own offset; positions off the box hold zeros.
+template <class TP, int D>
+constexpr int kTailVerts = D <= 3 ? 2 : 1;
+template <class TP, int D>
+constexpr int kTailPitch = D == 1 ? 2050 : D == 2 ? 47 : D == 3 ? 14 : 7;
+template <class TP>
+struct TailLevel {
+  Box box;
+  const TP* A;
+  const TP* dinv;
+  const uint8_t* alive;
+  // LDS values: two iterates with zeros around them (a stencil read past the box
+  // meets a zero coefficient and one of them), and below the first level the
+  // right-hand side, dinv and the + diagonals
+  int x, y, r, d, a;
+};
+template <class TP>
+struct Tail {
+  TailLevel<TP> l[TAIL_LEVELS];
+  const TP* cinv;
+  int levels, sweeps;
+  int c, total;  // the dense inverse in LDS (-1: read from memory); LDS values in use
+};
+
+// rc = P^T e on the live vertices of the coarser box
+template <class TP, int D>
+__device__ __forceinline__ void tail_restrict(const TailLevel<TP>& l, const TailLevel<TP>& c, const TP* e, TP* rc) {
+  constexpr int H = (1 << D) - 1;
+  for (int w = threadIdx.x; w < c.box.nb; w += TAIL_TPB) {
+    TP acc = TP(0);
+    if (c.alive[w]) {
+      int wc[D];
+      int k = w;
+#pragma unroll
+      for (int a = 0; a < D; ++a) {
+        wc[a] = 2 * (k % (c.box.g + 1));
+        k /= c.box.g + 1;
+      }
+#pragma unroll
+      for (int s = 0; s <= 2 * H; ++s) {
+        const int mask = s <= H ? s : s - H;
+        const int sg = s <= H ? 1 : -1;
+        bool in = true;
+        int j = 0;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+          const int f = wc[a] + ((mask >> a) & 1) * sg;
+          in = in && f >= 0 && f <= l.box.g;
+          j += f * l.box.st[a];
+        }
+        acc += (in ? (s == 0 ? TP(1) : TP(0.5)) : TP(0)) * e[in ? j : 0];
+      }
+    }
+    rc[w] = acc;
+  }
+}
+
+// (P xc)(i) of a live vertex
+template <class TP, int D>
+__device__ __forceinline__ TP tail_prolong(const TailLevel<TP>& l, const TailLevel<TP>& c, const TP* xc, int i) {
+  int k = i, lo = 0, hi = 0;
+  bool odd = false;
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    const int f = k % (l.box.g + 1);
+    k /= l.box.g + 1;
+    lo += (f >> 1) * c.box.st[a];
+    hi += ((f >> 1) + (f & 1)) * c.box.st[a];
+    odd = odd || (f & 1);
+  }
+  return odd ? TP(0.5) * (xc[lo] + xc[hi]) : xc[lo];
+}
+
+// A sweep (out = x + dinv (r - A x)) or, with RES, the residual on live rows
+// (0 on dead ones) of a level whose operator is in LDS.
+template <class TP, int D, bool RES>
+__device__ __forceinline__ void tail_sweep(const TailLevel<TP>& l, const TP* sm, const TP* x, TP* out) {
+  constexpr int H = (1 << D) - 1;
+  const int nb = l.box.nb;
+  const TP* A = sm + l.a;
+  for (int i = threadIdx.x; i < nb; i += TAIL_TPB) {
+    const TP xi = x[i];
+    TP acc = A[i] * xi;
+#pragma unroll
+    for (int m = 1; m <= H; ++m) {
+      const int o = stencil_offset<D>(m, l.box.st);
+      acc += A[m * nb + i] * x[i + o];
+      if (i >= o) acc += A[m * nb + i - o] * x[i - o];
+    }
+    const TP di = sm[l.d + i];
+    const TP res = sm[l.r + i] - acc;
+    out[i] = RES ? (di != TP(0) ? res : TP(0)) : xi + di * res;
+  }
+  __syncthreads();
+}
+
+template <class TP, int D, int K, int P>
+__global__ void __launch_bounds__(TAIL_TPB) k_st_tail(Tail<TP> t, const TP* __restrict__ r0,
+                                                      TP* __restrict__ x0, const MinresS* S) {
+  constexpr int H = (1 << D) - 1;
+  if (skip(S)) return;
+  __shared__ __align__(16) unsigned char raw[TAIL_LDS];
+  TP* sm = reinterpret_cast<TP*>(raw);
+  const int tid = threadIdx.x;
+  const int v = blockIdx.x;
+  const TailLevel<TP>& f = t.l[0];
+  const int nb = f.box.nb;
+  // the first level's operator, smoother and right-hand side, and the place of each vertex
+  TileRow<TP, D> w[K];
+  TP r[K];
+  int pos[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = tid + k * TAIL_TPB;
+    const unsigned j = i < nb ? (unsigned)i : 0u;
+    tile_row<TP, D>(w[k], f.A, f.dinv, f.box, j, i < nb);
+    r[k] = (r0 + (int64_t)v * nb)[j];
+    pos[k] = 0;
+    int c = (int)j;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      pos[k] += c % (f.box.g + 1) * tail_stride<D, P>(a);
+      c /= f.box.g + 1;
+    }
+  }
+#pragma unroll 4
+  for (int i = tid; i < t.c; i += TAIL_TPB) sm[i] = TP(0);  // the vectors and the positions off the boxes
+  __syncthreads();
+  // the other levels' operators and the dense inverse
+  for (int q = 1; q + 1 < t.levels; ++q) {
+    const TailLevel<TP>& l = t.l[q];
+    for (int i = tid; i < l.box.nb; i += TAIL_TPB) sm[l.d + i] = l.dinv[i];
+#pragma unroll 8
+    for (int i = tid; i < (H + 1) * l.box.nb; i += TAIL_TPB) sm[l.a + i] = l.A[i];
+  }
+  const TailLevel<TP>& last = t.l[t.levels - 1];
+  const int nl = last.box.nb;
+  const bool dense_lds = t.total > t.c;
+  if (dense_lds) {
+#pragma unroll 8
+    for (int i = tid; i < nl * nl; i += TAIL_TPB) sm[t.c + i] = t.cinv[i];
+  }
+  // the sweep family on the first level, its operator in registers
+  const auto sweep = [&](bool residual, const TP* x, TP* out) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (tid + k * TAIL_TPB < nb) {
+        const TP* xp = x + pos[k];
+        const TP res = tile_residual<TP, D, P>(w[k], r[k], xp);
+        out[pos[k]] = residual ? (w[k].d != TP(0) ? res : TP(0)) : *xp + w[k].d * res;
+      }
+    }
+    __syncthreads();
+  };
+  // down. Each level's iterate before the correction ends in its x, the residual in its y.
+  {
+    TP* x = sm + ((t.sweeps & 1) ? f.x : f.y);
+    TP* y = sm + ((t.sweeps & 1) ? f.y : f.x);
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (tid + k * TAIL_TPB < nb) x[pos[k]] = w[k].d * r[k];
+    __syncthreads();
+    for (int s = 1; s < t.sweeps; ++s) {
+      sweep(false, x, y);
+      TP* z = x;
+      x = y;
+      y = z;
+    }
+    sweep(true, x, y);
+    const TailLevel<TP>& c = t.l[1];
+    for (int w = tid; w < c.box.nb; w += TAIL_TPB) {
+      const TP* e = y;
+      int k = w;
+#pragma unroll
+      for (int a = 0; a < D; ++a) {
+        e += 2 * (k % (c.box.g + 1)) * tail_stride<D, P>(a);
+        k /= c.box.g + 1;
+      }
+      TP acc = TP(0);
+#pragma unroll
+      for (int m = 1; m <= H; ++m) acc += e[tail_offset<D, P>(m)] + e[-tail_offset<D, P>(m)];
+      acc = e[0] + TP(0.5) * acc;
+      sm[c.r + w] = c.alive[w] ? acc : TP(0);
+    }
+    __syncthreads();
+  }
+  for (int q = 1; q + 1 < t.levels; ++q) {
+    const TailLevel<TP>& l = t.l[q];
+    TP* x = sm + ((t.sweeps & 1) ? l.x : l.y);
+    TP* y = sm + ((t.sweeps & 1) ? l.y : l.x);
+    for (int i = tid; i < l.box.nb; i += TAIL_TPB) x[i] = sm[l.d + i] * sm[l.r + i];
+    __syncthreads();
+    for (int s = 1; s < t.sweeps; ++s) {
+      tail_sweep<TP, D, false>(l, sm, x, y);
+      TP* z = x;
+      x = y;
+      y = z;
+    }
+    tail_sweep<TP, D, true>(l, sm, x, y);
+    tail_restrict<TP, D>(l, t.l[q + 1], y, sm + t.l[q + 1].r);
+    __syncthreads();
+  }
+  // the coarsest level by its dense inverse, 8 lanes a row
+  {
+    const TP* rl = sm + last.r;
+    const int lane = tid & 7;
+    for (int i0 = 0; i0 < nl; i0 += TAIL_TPB / 8) {  // uniform trip count: the shuffles see whole groups
+      const int i = i0 + (tid >> 3);
+      TP acc = TP(0);
+      if (i < nl) {
+        if (dense_lds)
+          for (int j = lane; j < nl; j += 8) acc += sm[t.c + i * nl + j] * rl[j];
+        else
+          for (int j = lane; j < nl; j += 8) acc += t.cinv[i * nl + j] * rl[j];
+      }
+#pragma unroll
+      for (int off = 4; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+      if (i < nl && lane == 0) sm[last.x + i] = acc;
+    }
+    __syncthreads();
+  }
+  // up: the correction on x, post-smoothing
+  const TP* xc = sm + last.x;
+  for (int q = t.levels - 2; q >= 1; --q) {
+    const TailLevel<TP>& l = t.l[q];
+    TP* x = sm + l.x;
+    TP* y = sm + l.y;
+    for (int i = tid; i < l.box.nb; i += TAIL_TPB)
+      if (sm[l.d + i] != TP(0)) x[i] += tail_prolong<TP, D>(l, t.l[q + 1], xc, i);
+    __syncthreads();
+    for (int s = 0; s < t.sweeps; ++s) {
+      tail_sweep<TP, D, false>(l, sm, x, y);
+      TP* z = x;
+      x = y;
+      y = z;
+    }
+    xc = x;
+  }
+  {
+    TP* x = sm + f.x;
+    TP* y = sm + f.y;
+    const TailLevel<TP>& c = t.l[1];
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (tid + k * TAIL_TPB < nb && w[k].d != TP(0)) {
+        int q = pos[k], lo = 0, hi = 0;
+        bool odd = false;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+          const int u = q % P;  // a constant pitch: no division
+          q /= P;
+          lo += (u >> 1) * c.box.st[a];
+          hi += ((u + 1) >> 1) * c.box.st[a];
+          odd = odd || (u & 1);
+        }
+        x[pos[k]] += odd ? TP(0.5) * (xc[lo] + xc[hi]) : xc[lo];
+      }
+    __syncthreads();
+    for (int s = 0; s < t.sweeps; ++s) {
+      sweep(false, x, y);
+      TP* z = x;
+      x = y;
+      y = z;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (tid + k * TAIL_TPB < nb) x0[(int64_t)v * nb + tid + k * TAIL_TPB] = x[pos[k]];
   }
 }
 
@@ -432,13 +992,13 @@ __global__ void k_st_galerkin(const double* __restrict__ Af, const uint8_t* __re
 // ---------------------------------------------------------------------------
 // HX transfers between the KKT vector and the level-0 slots
 // ---------------------------------------------------------------------------
-// y[row * nv + slot0 + v] = sum_p val[p * C + v] x[col[p]] for v < C; LPR
+// y[(slot0 + v) * ny + row] = sum_p val[p * C + v] x[col[p]] for v < C; LPR
 // lanes share a row (entries strided over them, summed by shuffles).
 template <class TX, class TP, int LPR>
 __global__ void __launch_bounds__(TPB) k_hx_gather(const int64_t* __restrict__ rp,
                                                    const int32_t* __restrict__ col,
                                                    const TP* __restrict__ val, int C,
-                                                   const TX* __restrict__ x, TP* __restrict__ y, int nv,
+                                                   const TX* __restrict__ x, TP* __restrict__ y, int64_t ny,
                                                    int slot0, int64_t nrows, const MinresS* S) {
   if (skip(S)) return;
   const int64_t gid = xcd_block() * (int64_t)blockDim.x + threadIdx.x;
@@ -465,18 +1025,18 @@ __global__ void __launch_bounds__(TPB) k_hx_gather(const int64_t* __restrict__ r
     }
   }
   if (row < nrows && lane == 0)
-    for (int v = 0; v < C; ++v) y[row * nv + slot0 + v] = acc[v];
+    for (int v = 0; v < C; ++v) y[(slot0 + v) * ny + row] = acc[v];
 }
 
 // y[row] = (a ? a[row] b[row] : add ? y[row] : 0)
 //          + sum_p sum_v val[p * C + v] X(col[p], v),
-// X(c, v) = x0[c * nv + slot0 + v], except X(c, 0) = x0[..] + dl[c] r0[..]
+// X(c, v) = x0[(slot0 + v) * nx + c], except X(c, 0) = x0[..] + dl[c] r0[..]
 // when `grad` (the grade-0 term S_0 t + V t of the gradient correction).
 template <class TP, class TA, class TB>
 __global__ void __launch_bounds__(TPB) k_hx_out(const int64_t* __restrict__ rp, const int32_t* __restrict__ col,
                                                 const TP* __restrict__ val, int C, int grad,
                                                 const TP* __restrict__ x0, const TP* __restrict__ r0,
-                                                const TP* __restrict__ dl, int nv, int slot0,
+                                                const TP* __restrict__ dl, int64_t nx, int slot0,
                                                 const TA* __restrict__ a, const TB* __restrict__ b,
                                                 TP* __restrict__ y, int64_t nrows, int add, const MinresS* S) {
   if (skip(S)) return;
@@ -484,11 +1044,11 @@ __global__ void __launch_bounds__(TPB) k_hx_out(const int64_t* __restrict__ rp, 
   if (i >= nrows) return;
   TP acc = a ? (TP)a[i] * (TP)b[i] : (add ? y[i] : TP(0));
   for (int64_t p = rp[i]; p < rp[i + 1]; ++p) {
-    const int64_t base = (int64_t)col[p] * nv + slot0;
+    const int64_t base = slot0 * nx + col[p];
     TP x = x0[base];
     if (grad) x += dl[col[p]] * r0[base];
     acc += val[p * C] * x;
-    for (int v = 1; v < C; ++v) acc += val[p * C + v] * x0[base + v];
+    for (int v = 1; v < C; ++v) acc += val[p * C + v] * x0[base + v * nx];
   }
   y[i] = acc;
 }
@@ -497,25 +1057,25 @@ __global__ void __launch_bounds__(TPB) k_hx_out(const int64_t* __restrict__ rp, 
 // v0 < v1 (box vertices), D_0 has -1 at v0 and +1 at v1 and Pi_1 the same D
 // values eh = (x(v1) - x(v0)) / 2 at both ends:
 //   z[e] = s[e] r[e] + (G(v1) - G(v0)) + sum_c eh[e, c] (X_c(v0) + X_c(v1)),
-// G(v) = x0[v, slot0] + dl[v] r0[v, slot0] and X_c(v) = x0[v, slot0 + 1 + c].
+// G(v) = x0[slot0, v] + dl[v] r0[slot0, v] and X_c(v) = x0[slot0 + 1 + c, v].
 // Vertices that are not unknowns hold zeros in every slot, so both ends are
 // always read.
 template <class TP, class TB, int D>
 __global__ void __launch_bounds__(TPB) k_hx_out_edge(const int32_t* __restrict__ ev, const TP* __restrict__ eh,
                                                      const TP* __restrict__ x0, const TP* __restrict__ r0,
-                                                     const TP* __restrict__ dl, int nv, int slot0,
+                                                     const TP* __restrict__ dl, int64_t nx, int slot0,
                                                      const TP* __restrict__ s, const TB* __restrict__ r,
                                                      TP* __restrict__ z, int64_t nrows, const MinresS* S) {
   if (skip(S)) return;
   const int64_t e = xcd_block() * (int64_t)blockDim.x + threadIdx.x;
   if (e >= nrows) return;
   const int v0 = ev[2 * e], v1 = ev[2 * e + 1];
-  const TP* a = x0 + (int64_t)v0 * nv + slot0;
-  const TP* b = x0 + (int64_t)v1 * nv + slot0;
+  const TP* a = x0 + slot0 * nx + v0;
+  const TP* b = x0 + slot0 * nx + v1;
   TP acc = s[e] * (TP)r[e];
-  acc += (b[0] + dl[v1] * r0[(int64_t)v1 * nv + slot0]) - (a[0] + dl[v0] * r0[(int64_t)v0 * nv + slot0]);
+  acc += (b[0] + dl[v1] * r0[slot0 * nx + v1]) - (a[0] + dl[v0] * r0[slot0 * nx + v0]);
 #pragma unroll
-  for (int c = 0; c < D; ++c) acc += eh[e * D + c] * (a[1 + c] + b[1 + c]);
+  for (int c = 0; c < D; ++c) acc += eh[e * D + c] * (a[(1 + c) * nx] + b[(1 + c) * nx]);
   z[e] = acc;
 }
 
@@ -1007,6 +1567,8 @@ struct Hx {
   DBuf<double> res64, d64, zc64, w64;
   DBuf<float> res32, d32, zc32, w32;
   int64_t bytes32 = 0, launches = 0;
+  // the first level of the cycle's one-launch end (k_st_tail), in FP32 and FP64
+  size_t tail32 = 0, tail64 = 0;
   // the spectrum estimate's launches, captured once and replayed per refresh
   bool use_graph = true;         // replay the estimate from a graph (else launch one by one)
   bool lz_direct_ready = false;  // the start vector is on the device
@@ -1539,6 +2101,8 @@ void smoother_diag(Hx& h, const KktSystem& s) {
 
 namespace {
 void hx_spectrum(Hx& h);
+template <class TP>
+size_t tail_start(const Hx& h);
 
 // The KKT preconditioner matrix P (blockdiag(hdif_gram(k-1), hdif_gram(k)))
 // the Chebyshev steps multiply by, and its symmetric FP32 copy.
@@ -1825,6 +2389,8 @@ Hx* hx_create(Geom& g, int bc, int k, const KktSystem& s, int sweeps, int cheb_m
     for (const XCsr* x : {&b.g_main, &b.o_main, &b.g_t, &b.g_tl, &b.o_ul, &b.o_d})
       if (x->C > MAXC) return no("too many components per transfer entry");
   h->nv = slot;
+  h->tail32 = tail_start<float>(*h);
+  h->tail64 = tail_start<double>(*h);
   alloc_slots(ctx, *h);
   h->zt64.alloc(ctx, std::max<int64_t>(h->N, 1));
   h->zt32.alloc(ctx, std::max<int64_t>(h->N, 1));
@@ -1858,7 +2424,7 @@ Hx* hx_create(Geom& g, int bc, int k, const KktSystem& s, int sweeps, int cheb_m
     const int64_t nbv = (int64_t)l.box.nb * h->nv;
     if (i + 1 < h->L.size()) {
       bytes += (int64_t)(2 * h->sweeps) * ((int64_t)(NS / 2 + 1) * l.box.nb * 4 + 12 * nbv) + 16 * nbv;
-      launches += 2 + 2 * h->sweeps;
+      if (i < h->tail32) launches += 2 + 2 * h->sweeps;
     } else {
       bytes += (int64_t)l.box.nb * l.box.nb * 4;
       launches += 1;
@@ -1971,8 +2537,90 @@ struct Sel<float> {
   static float* w(Hx& h) { return h.w32.p; }
 };
 
-// One V-cycle on level i with its rhs in r(i); returns the buffer holding
-// the result (x(i) or y(i)).
+// k_st_tail's levels and LDS for the cycle from level i on.
+template <class TP, int D>
+Tail<TP> tail_layout(const Hx& h, size_t i) {
+  using X = Sel<TP>;
+  constexpr int P = kTailPitch<TP, D>;
+  Tail<TP> t{};
+  t.levels = (int)(h.L.size() - i);
+  t.sweeps = h.sweeps;
+  t.cinv = X::cinv(h);
+  int at = 0;
+  const auto take = [&](int n) {
+    const int o = at;
+    at += n;
+    return o;
+  };
+  for (int k = 0; k < t.levels && k < TAIL_LEVELS; ++k) {
+    const MgLevel& m = h.L[i + k];
+    TailLevel<TP>& l = t.l[k];
+    l = {m.box, X::A(m), X::dinv(m), m.alive.p};
+    const int nb = m.box.nb;
+    if (k + 1 == t.levels) {
+      l.x = take(nb);
+      l.r = take(nb);
+      break;
+    }
+    // two iterates with room for a stencil's reach before, between and after them
+    int pad = 0;
+    for (int a = 0; a < h.d; ++a) pad += k ? m.box.st[a] : tail_stride<D, P>(a);
+    const int len = k ? nb : tail_stride<D, P>(D);
+    l.x = take(pad) + pad;
+    take(len);
+    l.y = take(pad) + pad;
+    take(len + pad);
+    if (k) {
+      l.r = take(nb);
+      l.d = take(nb);
+      l.a = take((1 << h.d) * nb);
+    }
+  }
+  const int nl = h.L.back().box.nb;
+  t.c = t.total = at;
+  if ((int64_t)(at + (int64_t)nl * nl) * (int64_t)sizeof(TP) <= TAIL_LDS) t.total += nl * nl;
+  return t;
+}
+
+// The first level of the cycle's one-launch end: the finest one whose vertices
+// fit the registers and the pitch and, with the coarser levels, the LDS; the
+// number of levels when there is none with a level below it.
+template <class TP, int D>
+size_t tail_start_d(const Hx& h) {
+  const size_t n = h.L.size();
+  for (size_t i = 0; i + 1 < n; ++i)
+    if (n - i <= (size_t)TAIL_LEVELS && h.L[i].box.nb <= TAIL_TPB * kTailVerts<TP, D> &&
+        h.L[i].box.g + 3 <= kTailPitch<TP, D> &&
+        (int64_t)tail_layout<TP, D>(h, i).total * (int64_t)sizeof(TP) <= TAIL_LDS)
+      return i;
+  return n;
+}
+template <class TP>
+size_t tail_start(const Hx& h) {
+  switch (h.d) {
+    case 1: return tail_start_d<TP, 1>(h);
+    case 2: return tail_start_d<TP, 2>(h);
+    case 3: return tail_start_d<TP, 3>(h);
+    default: return tail_start_d<TP, 4>(h);
+  }
+}
+
+// The tiles of a level: `down` cover the coarser box, `up` its own.
+struct LevelTiles {
+  int d, nd, nu, down, up;
+  LevelTiles(int dim, const Box& f, const Box& c) : d(dim) {
+    const int T = d == 1 ? kTile<1> : d == 2 ? kTile<2> : kTile<3>;
+    nd = (c.g + T) / T;
+    nu = (f.g + 2 * T) / (2 * T);
+    down = cpow(nd, d);
+    up = cpow(nu, d);
+  }
+  // whether the level takes k_st_down / k_st_up: two sweeps, and no more
+  // workgroups than run at once (two a CU in 3D; 2D's use fewer registers and
+  // recompute less)
+  bool use(const Hx& h) const { return d <= 3 && h.sweeps == 2 && std::max(down, up) * h.nv <= (d == 3 ? 512 : 2048); }
+};
+
 template <class TP, int D, bool FINE>
 void sweep_launch(Enq& q, int mode, const MgLevel& l, const TP* A, const TP* dinv, const TP* r, const TP* x,
                   TP* out, unsigned nv, const MinresS* S) {
@@ -1992,6 +2640,11 @@ TP* vcycle(Enq& q, Hx& h, size_t i, const MinresS* S) {
   MgLevel& l = h.L[i];
   const unsigned nv = (unsigned)h.nv;
   const int64_t nbv = (int64_t)l.box.nb * nv;
+  if (i == (std::is_same_v<TP, float> ? h.tail32 : h.tail64)) {
+    Tail<TP> t = tail_layout<TP, D>(h, i);
+    q(k_st_tail<TP, D, kTailVerts<TP, D>, kTailPitch<TP, D>>, nv, TAIL_TPB, t, (const TP*)X::r(l), X::x(l), S);
+    return X::x(l);
+  }
   if (i + 1 == h.L.size()) {
     q(k_st_dense<TP>, (unsigned)l.box.nb, TPB, X::cinv(h), (const TP*)X::r(l), X::x(l), l.box.nb, h.nv, S);
     return X::x(l);
@@ -2002,6 +2655,17 @@ TP* vcycle(Enq& q, Hx& h, size_t i, const MinresS* S) {
   const TP* r = X::r(l);
   const TP* A = X::A(l);
   const TP* dinv = X::dinv(l);
+  if constexpr (D <= 3) {
+    const LevelTiles g(D, l.box, c.box);
+    if (g.use(h)) {
+      q(k_st_down<TP, D>, dim3((unsigned)g.down, nv), TILE_TPB, A, dinv, r, x, X::r(c), (const uint8_t*)c.alive.p,
+        l.box, c.box, g.nd, S);
+      const TP* xc = vcycle<TP, D>(q, h, i + 1, S);
+      q(k_st_up<TP, D>, dim3((unsigned)g.up, nv), TILE_TPB, A, dinv, r, (const TP*)x, xc, y, l.box, c.box, g.nu,
+        S);
+      return y;
+    }
+  }
   auto sweep = [&](int mode, TP* out) {
     if (i == 0)
       sweep_launch<TP, D, true>(q, mode, l, A, dinv, r, x, out, nv, S);
@@ -2032,14 +2696,14 @@ TP* vcycle(Enq& q, Hx& h, size_t i, const MinresS* S) {
 }
 
 template <class TX, class TP>
-void gather(Enq& q, const XCsr& g, const TX* x, TP* y, int nv, int slot0, const MinresS* S) {
+void gather(Enq& q, const XCsr& g, const TX* x, TP* y, int64_t ny, int slot0, const MinresS* S) {
   using X = Sel<TP>;
   const int64_t nr = g.m.nrows;
   if (g.avg_row >= 6.0)
-    q(k_hx_gather<TX, TP, 4>, grid_for(nr * 4), TPB, g.m.row_ptr.p, g.m.col.p, X::v(g), g.C, x, y, nv, slot0,
+    q(k_hx_gather<TX, TP, 4>, grid_for(nr * 4), TPB, g.m.row_ptr.p, g.m.col.p, X::v(g), g.C, x, y, ny, slot0,
       nr, S);
   else
-    q(k_hx_gather<TX, TP, 1>, grid_for(nr), TPB, g.m.row_ptr.p, g.m.col.p, X::v(g), g.C, x, y, nv, slot0, nr,
+    q(k_hx_gather<TX, TP, 1>, grid_for(nr), TPB, g.m.row_ptr.p, g.m.col.p, X::v(g), g.C, x, y, ny, slot0, nr,
       S);
 }
 
@@ -2050,14 +2714,14 @@ void hx_core_d(Enq& q, Hx& h, const TIN* r, const MinresS* S) {
   MgLevel& l0 = h.L[0];
   TP* slots = X::r(l0);
   TP* zt = X::zt(h);
-  const int nv = h.nv;
+  const int64_t nx = l0.box.nb;
   for (HxBlock& b : h.blocks) {
     const TIN* rb = r + b.off;
     if (b.j == 2) {
-      gather<TIN, TP>(q, b.g_t, rb, X::t(b), 1, 0, S);
-      gather<TP, TP>(q, b.g_tl, (const TP*)X::t(b), slots, nv, b.slot_tl, S);
+      gather<TIN, TP>(q, b.g_t, rb, X::t(b), nx, 0, S);
+      gather<TP, TP>(q, b.g_tl, (const TP*)X::t(b), slots, nx, b.slot_tl, S);
     }
-    gather<TIN, TP>(q, b.g_main, rb, slots, nv, b.slot_main, S);
+    gather<TIN, TP>(q, b.g_main, rb, slots, nx, b.slot_main, S);
   }
   const TP* xs = vcycle<TP, D>(q, h, 0, S);
   for (HxBlock& b : h.blocks) {
@@ -2068,19 +2732,19 @@ void hx_core_d(Enq& q, Hx& h, const TIN* r, const MinresS* S) {
     if (b.j == 2) {
       const XCsr& ul = b.o_ul;
       q(k_hx_out<TP, TP, TP>, grid_for(ul.m.nrows), TPB, ul.m.row_ptr.p, ul.m.col.p, X::v(ul), ul.C, 0, xs,
-        (const TP*)slots, X::dinv(l0), nv, b.slot_tl, X::sl(b), (const TP*)X::t(b), X::u(b), ul.m.nrows, 0, S);
+        (const TP*)slots, X::dinv(l0), nx, b.slot_tl, X::sl(b), (const TP*)X::t(b), X::u(b), ul.m.nrows, 0, S);
       const XCsr& od = b.o_d;
       q(k_hx_out<TP, TP, TIN>, grid_for(od.m.nrows), TPB, od.m.row_ptr.p, od.m.col.p, X::v(od), od.C, 0,
-        (const TP*)X::u(b), (const TP*)nullptr, (const TP*)nullptr, 1, 0, sb, rb, zb, od.m.nrows, 0, S);
+        (const TP*)X::u(b), (const TP*)nullptr, (const TP*)nullptr, nx, 0, sb, rb, zb, od.m.nrows, 0, S);
       q(k_hx_out<TP, TP, TIN>, grid_for(om.m.nrows), TPB, om.m.row_ptr.p, om.m.col.p, X::v(om), om.C, 0, xs,
-        (const TP*)slots, X::dinv(l0), nv, b.slot_main, (const TP*)nullptr, (const TIN*)nullptr, zb,
+        (const TP*)slots, X::dinv(l0), nx, b.slot_main, (const TP*)nullptr, (const TIN*)nullptr, zb,
         om.m.nrows, 1, S);
     } else if (b.edge_free) {
       q(k_hx_out_edge<TP, TIN, D>, grid_for(b.n), TPB, (const int32_t*)b.ev.p, X::eh(b), xs, (const TP*)slots,
-        X::dinv(l0), nv, b.slot_main, sb, rb, zb, b.n, S);
+        X::dinv(l0), nx, b.slot_main, sb, rb, zb, b.n, S);
     } else {
       q(k_hx_out<TP, TP, TIN>, grid_for(om.m.nrows), TPB, om.m.row_ptr.p, om.m.col.p, X::v(om), om.C,
-        b.j == 1 ? 1 : 0, xs, (const TP*)slots, X::dinv(l0), nv, b.slot_main, sb, rb, zb, om.m.nrows, 0, S);
+        b.j == 1 ? 1 : 0, xs, (const TP*)slots, X::dinv(l0), nx, b.slot_main, sb, rb, zb, om.m.nrows, 0, S);
     }
   }
 }

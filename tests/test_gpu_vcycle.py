@@ -1,0 +1,48 @@
+"""The V-cycle's launch forms on the GPU against the oracle's cycle: a level in
+two launches (tiles with halos), the coarse end in one workgroup per slot, and
+the kernels of one sweep each, at box sizes around the tiles' and the
+workgroup's edges."""
+import numpy as np
+import pytest
+
+import formoniq_amd as fa
+from oracle import oracle as o
+
+from _common import both
+
+pytestmark = pytest.mark.gpu
+
+# (d, n, k, relative, sweeps): two-launch levels from 13^3 and 46^2 vertices on, partial last
+# tiles, odd grids whose coarse box overhangs, a whole cycle in one launch (the largest and
+# one smaller), 4D (no tiles), one and three sweeps (no tiles; the iterates change buffers)
+CASES = [(1, 900, 0, True, 2), (1, 5000, 0, True, 2), (2, 44, 1, False, 2), (2, 45, 1, True, 2), (2, 66, 0, True, 2),
+         (2, 97, 1, False, 2), (3, 11, 1, False, 2), (3, 12, 1, True, 2), (3, 13, 2, True, 2), (3, 15, 1, False, 2),
+         (3, 17, 0, True, 2), (3, 26, 0, True, 2), (4, 4, 1, False, 2), (2, 50, 1, False, 3), (3, 12, 1, False, 1),
+         (3, 13, 1, True, 3)]
+
+
+@pytest.mark.parametrize("d,n,k,rel,sweeps", CASES)
+def test_cycle_forms_match_the_oracle(d, n, k, rel, sweeps):
+    """One block application (m = 1) in FP64 to 1e-10 of its largest entry and in
+    FP32 to 1e-5, the bounds of the other application tests (sums of at most 31
+    terms in another order), where the grid is coarse enough for the latter: in
+    FP32 a residual is rounded to 6e-8 of A x, and the coarse correction of its
+    smooth part amplifies that by up to the condition number of D^-1 A, about
+    4 n^2 / pi^2."""
+    ocx, oL, gcx, geo, cells, coords = both(d, n, 0.05, seed=n)
+    gc = fa.WhitneyComplex(geo, relative=rel)
+    opts = dict(preconditioner=fa.PC_MULTIGRID, cheb_degree=1, mg_sweeps=sweeps)
+    prob = fa.Problem(gc, k, fa.solve_opts(precision=fa.FP64, **opts))
+    prob.assemble()
+    ns, nu, nh = prob.sizes
+    oc = o.WhitneyComplex(ocx, oL, relative=rel)
+    r = np.sin(np.arange(ns + nu + nh) * 0.7 + 0.3)
+    want = o.hx_block_preconditioner(oc, coords, k, n, nh, sweeps=sweeps, cheb_m=1)(r)
+    scale = np.abs(want).max()
+    got = prob.apply_preconditioner(r, precision=fa.FP64)
+    assert np.abs(got - want).max() <= 1e-10 * scale, np.abs(got - want).max() / scale
+    got32 = fa.Problem(gc, k, fa.solve_opts(**opts)).apply_preconditioner(r, precision=fa.FP64_PC32)
+    tol32 = max(1e-5, 6e-8 * 0.4 * n * n)
+    assert np.abs(got32 - want).max() <= tol32 * scale, np.abs(got32 - want).max() / scale
+    again = prob.apply_preconditioner(r, precision=fa.FP64)
+    np.testing.assert_array_equal(again, got)
