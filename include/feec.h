@@ -127,8 +127,9 @@ typedef struct feec_solve_opts {
  *   under refinement. It needs a Kuhn-grid mesh numbered as feec_kuhn_grid numbers it, a
  *   geometry from Euclidean coordinates and grade <= 2; otherwise FEEC_E_UNSUPPORTED.
  * FEEC_PC_CHEBYSHEV: a Chebyshev-Jacobi polynomial of degree cheb_degree on each block.
- * FEEC_PC_AUTO: multigrid where it applies and the system is not small (at least 20,000
- *   KKT rows), else Chebyshev. Batched solves (feec_batch_run) always run Chebyshev. */
+ * FEEC_PC_AUTO: multigrid where it applies, else Chebyshev; below 20,000 KKT rows also
+ *   Chebyshev where cheb_degree >= 0 asks for a degree, and for grade 2 of the relative
+ *   complex. Batched solves (feec_batch_run) always run Chebyshev. */
 typedef enum {
   FEEC_PC_AUTO = 0,
   FEEC_PC_CHEBYSHEV = 1,

@@ -202,3 +202,37 @@ def test_c2_full_size_multigrid():
     assert np.linalg.norm(u64 - u_ch) <= 1e-8 * np.linalg.norm(u_ch)
     print("64^3 iterations: multigrid FP64_PC32", rep_mg.iters, "FP64", rep64.iters,
           "chebyshev", rep_ch.iters)
+
+
+@pytest.mark.parametrize("d,n,k,rel", [(1, 9, 0, True), (2, 2, 1, False), (2, 3, 0, True), (2, 7, 0, False),
+                                       (2, 16, 1, True), (2, 9, 2, False), (2, 8, 2, True), (3, 2, 1, False),
+                                       (3, 5, 0, True), (3, 4, 2, False), (3, 4, 2, True), (4, 2, 1, False),
+                                       (4, 3, 0, True), (3, 3, 3, False)])
+def test_auto_on_small_grids(d, n, k, rel):
+    """PC_AUTO on systems below 20,000 rows: multigrid wherever PC_MULTIGRID can be
+    built, except grade 2 of the relative complex, the polynomial otherwise and
+    where a degree is asked for; the solution is the polynomial's to the solve
+    tolerance (residuals of 1e-10 times a condition below 1e4 on these grids)."""
+    _, _, gcx, geo, _, _ = both(d, n, 0.05, seed=n)
+    wc = fa.WhitneyComplex(geo, relative=rel)
+    f = fa.normal_vector(gcx.nsimplices(k), 2)
+    try:
+        fa.Problem(wc, k, mg_opts()).assemble()
+        can = True
+    except fa.FeecError as e:
+        assert e.name == "FEEC_E_UNSUPPORTED"
+        can = False
+    auto = fa.Problem(wc, k)
+    auto.assemble()
+    want = can and not (k == 2 and rel)
+    assert auto.preconditioner()["format"].startswith("multigrid" if want else "sell64"), auto.preconditioner()
+    fixed = fa.Problem(wc, k, fa.solve_opts(cheb_degree=8))
+    fixed.assemble()
+    assert fixed.preconditioner()["format"].startswith("sell64")
+    poly = fa.Problem(wc, k, fa.solve_opts(preconditioner=fa.PC_CHEBYSHEV))
+    u = []
+    for prob in (auto, poly):
+        rep = prob.solve(f)
+        assert rep.converged and rep.residual <= 1e-10, rep.as_dict()
+        u.append(np.concatenate(prob.solution()[:2]))
+    assert np.linalg.norm(u[0] - u[1]) <= 1e-6 * np.linalg.norm(u[1])
