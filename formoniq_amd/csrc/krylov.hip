@@ -2862,17 +2862,55 @@ void axpy64(Ctx* ctx, const double* a, int64_t n, double s, double* x) {
 }
 
 // --- device-resident Jacobi CG -------------------------------------------------
-// The scalars live in device memory; the host reads them once per segment of
-// CG_SEG iterations, and iterations after convergence return at once.
+// Two launches an iteration (three on large systems). Every block sums the
+// partials of the launch before by itself, in the same fixed order, so alpha,
+// beta and the stopping test need no launch of one block of their own, and the
+// product forms its direction p = z + beta p as it gathers it. A scalar that one
+// launch reads and its block 0 also renews has a slot per parity of the
+// iteration. The host reads the state of a segment while the next one runs;
+// iterations after convergence return at once. The launches and the reads bound
+// it on small systems: with five launches an iteration and a read before each
+// next segment a mass solve of 31 k rows (32 iterations) took 907 us, now 731;
+// the leapfrog's, whose right-hand sides are on the device, 1,050 and 700 on
+// 111 k rows (36 iterations).
 struct CgS {
-  double rz, bnorm2, rtol2, alpha, beta, res2;
+  double rz[2];
+  long long iters[2];  // completed when the iteration of this parity starts
+  double bnorm2, rtol2, res2;
   long long iter, max_iters;
   int done;
   int pad;
 };
-constexpr int CG_SEG = 8;
+constexpr int CG_SEG = 8;  // even: a segment starts at parity 0
+constexpr int CG_RED = 1024, CG_ROWS = 2048;  // blocks at most: each block reads all partials
+// Rows up to which p is formed while gathered. Beyond, the two vectors miss the
+// caches (795 k rows: 59 us a product against 39) and p takes a launch of its own.
+constexpr int64_t CG_TWO_ROWS = 300000;
+constexpr int CG_RR = CG_RED, CG_PAP = 2 * CG_RED;  // places of the partials
+static_assert(CG_PAP + CG_ROWS <= 2 * NBLK, "CG partials fit their area");
 
-// x = 0, r = b, z = p = dinv b; partials r.z and b.b
+// The block's sums of a and b on every thread, over one barrier; sh: TPB / 32
+// doubles that nothing else uses.
+__device__ __forceinline__ void block_sums(double& a, double& b, double* sh) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    a += __shfl_xor(a, off, 64);
+    b += __shfl_xor(b, off, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    sh[threadIdx.x >> 6] = a;
+    sh[TPB / 64 + (threadIdx.x >> 6)] = b;
+  }
+  __syncthreads();
+  a = b = 0.0;
+#pragma unroll
+  for (int w = 0; w < TPB / 64; ++w) {
+    a += sh[w];
+    b += sh[TPB / 64 + w];
+  }
+}
+
+// x = 0, r = b, z = dinv b, p = 0; partials r.z and b.b
 __global__ void __launch_bounds__(TPB) k_cg_init(const double* __restrict__ b,
                                                  const double* __restrict__ dinv, int64_t n,
                                                  double* __restrict__ x, double* __restrict__ r,
@@ -2886,7 +2924,7 @@ __global__ void __launch_bounds__(TPB) k_cg_init(const double* __restrict__ b,
     x[i] = 0.0;
     r[i] = bi;
     z[i] = zi;
-    p[i] = zi;
+    p[i] = 0.0;
     rz += bi * zi;
     bb += bi * bi;
   }
@@ -2895,23 +2933,17 @@ __global__ void __launch_bounds__(TPB) k_cg_init(const double* __restrict__ b,
   const double t1 = block_reduce(bb, sh);
   if (threadIdx.x == 0) {
     part[blockIdx.x] = t0;
-    part[NBLK + blockIdx.x] = t1;
+    part[CG_RR + blockIdx.x] = t1;
   }
 }
 
 __global__ void k_cg_start(CgS* S, const double* part, int np, double rtol, long long max_iters) {
   __shared__ double sh[TPB / 64];
-  double a = 0.0, b = 0.0;
-  for (int i = threadIdx.x; i < np; i += blockDim.x) {
-    a += part[i];
-    b += part[NBLK + i];
-  }
-  const double rz = block_reduce(a, sh);
-  __syncthreads();
+  double b = 0.0;
+  for (int i = threadIdx.x; i < np; i += blockDim.x) b += part[CG_RR + i];
   const double bb = block_reduce(b, sh);
   if (threadIdx.x == 0) {
     CgS s{};
-    s.rz = rz;
     s.bnorm2 = bb;
     s.rtol2 = rtol * rtol;
     s.res2 = bb;
@@ -2921,107 +2953,185 @@ __global__ void k_cg_start(CgS* S, const double* part, int np, double rtol, long
   }
 }
 
-// ap = A p; partial p.ap
+// The scalars of the iteration's first launch: beta from the partials of r.z,
+// the stopping test on those of r.r (from the second iteration on; true: over).
+__device__ __forceinline__ bool cg_begin(CgS* S, const double* part, int np, int par, double* sh,
+                                         double& beta) {
+  const long long iter = S->iters[par], most = S->max_iters;
+  const double rz_old = S->rz[par], stop = S->rtol2 * S->bnorm2;
+  double rz = 0.0, rr = 0.0;
+  for (int i = threadIdx.x; i < np; i += TPB) {
+    rz += part[i];
+    rr += part[CG_RR + i];
+  }
+  block_sums(rz, rr, sh);
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  if (iter > 0 && (rr <= stop || iter >= most)) {
+    if (lead) {
+      S->res2 = rr;
+      S->iter = iter;
+      S->done = 1;
+    }
+    return true;
+  }
+  if (lead) {
+    S->rz[par ^ 1] = rz;
+    S->iters[par ^ 1] = iter + 1;
+  }
+  beta = iter > 0 ? rz / rz_old : 0.0;
+  return false;
+}
+
+// Rows of a block in the CG products: a contiguous share each, the shares dealt
+// so that an XCD's blocks are neighbours (the gathered vector then stays in
+// that XCD's L2). Blocks past the last row have none.
+__device__ __forceinline__ int64_t cg_share(int64_t n, int64_t& begin) {
+  constexpr int R = TPB / LANES;
+  const int64_t per = gridDim.x / XCDS, b = blockIdx.x;
+  const int64_t id = b < per * XCDS ? (b % XCDS) * per + b / XCDS : b;
+  const int64_t rows = ((n + R - 1) / R + gridDim.x - 1) / gridDim.x * R;
+  begin = id * rows;
+  return begin + rows < n ? begin + rows : n;
+}
+
+// ap = A p1; partial p1.ap. TWO: p1 = z + beta p0 is formed as it is gathered,
+// A z and A p0 apart, so that the first row's loads do not wait for beta.
+// Otherwise p1 is there (k_cg_dir) and z, p0 are not read.
+template <bool TWO>
 __global__ void __launch_bounds__(TPB) k_cg_spmv(const int64_t* __restrict__ rp,
                                                  const int32_t* __restrict__ col,
                                                  const double* __restrict__ val, int64_t n,
-                                                 const double* __restrict__ p,
-                                                 double* __restrict__ ap, const CgS* S,
-                                                 double* part) {
+                                                 const double* __restrict__ z,
+                                                 const double* __restrict__ p0,
+                                                 double* __restrict__ p1, double* __restrict__ ap,
+                                                 CgS* S, double* part, int np, int par) {
+  constexpr int U = SPMV_UNROLL;
   if (S->done) return;
-  __shared__ double sh[TPB / 64];
+  __shared__ double sh[TPB / 64], sh2[TPB / 32];
   const int lane = threadIdx.x % LANES;
-  const int64_t groups = (int64_t)gridDim.x * (TPB / LANES);
-  double loc = 0.0;
-  for (int64_t row = blockIdx.x * (int64_t)(TPB / LANES) + threadIdx.x / LANES; row < n;
-       row += groups) {
-    const double acc = row_dot<double>(rp, col, val, p, row, lane);
-    if (lane == 0) {
-      ap[row] = acc;
-      loc += p[row] * acc;
+  const auto sums = [&](int64_t row, double& az, double& aq) {
+    const double* __restrict__ x = TWO ? z : p1;
+    const int64_t end = rp[row + 1];
+    double t[U], w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) t[u] = w[u] = 0.0;
+    int64_t q = rp[row] + lane;
+    for (; q + (U - 1) * LANES < end; q += U * LANES) {
+      int32_t c[U];
+      double v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        c[u] = col[q + u * LANES];
+        v[u] = val[q + u * LANES];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        t[u] += v[u] * x[c[u]];
+        if (TWO) w[u] += v[u] * p0[c[u]];
+      }
     }
+#pragma unroll
+    for (int u = 0; u + 1 < U; ++u)
+      if (q + u * LANES < end) {
+        const int32_t c = col[q + u * LANES];
+        const double v = val[q + u * LANES];
+        t[u] += v * x[c];
+        if (TWO) w[u] += v * p0[c];
+      }
+    az = t[0];
+    aq = w[0];
+#pragma unroll
+    for (int u = 1; u < U; ++u) {
+      az += t[u];
+      aq += w[u];
+    }
+  };
+  int64_t begin;
+  const int64_t end = cg_share(n, begin);
+  int64_t row = begin + threadIdx.x / LANES;
+  double az = 0.0, aq = 0.0, beta = 0.0, loc = 0.0;
+  if (row < end) sums(row, az, aq);
+  if (TWO && cg_begin(S, part, np, par, sh2, beta)) return;
+  for (; row < end;) {
+    double acc = TWO ? az + beta * aq : az;
+#pragma unroll
+    for (int off = LANES / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, LANES);
+    if (lane == 0) {
+      const double pn = TWO ? z[row] + beta * p0[row] : p1[row];
+      if (TWO) p1[row] = pn;
+      ap[row] = acc;
+      loc += pn * acc;
+    }
+    row += TPB / LANES;
+    if (row < end) sums(row, az, aq);
   }
   const double t = block_reduce(loc, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = t;
+  if (threadIdx.x == 0) part[CG_PAP + blockIdx.x] = t;
 }
 
-__global__ void k_cg_alpha(CgS* S, const double* part, int np) {
+// p1 = z + beta p0
+__global__ void __launch_bounds__(TPB) k_cg_dir(const double* __restrict__ z, const double* __restrict__ p0,
+                                                double* __restrict__ p1, int64_t n, CgS* S, const double* part,
+                                                int np, int par) {
   if (S->done) return;
-  __shared__ double sh[TPB / 64];
-  double v = 0.0;
-  for (int i = threadIdx.x; i < np; i += blockDim.x) v += part[i];
-  const double pap = block_reduce(v, sh);
-  if (threadIdx.x == 0) S->alpha = S->rz / pap;
+  __shared__ double sh[TPB / 32];
+  double beta = 0.0;
+  if (cg_begin(S, part, np, par, sh, beta)) return;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    p1[i] = z[i] + beta * p0[i];
 }
 
-// x += alpha p, r -= alpha ap, z = dinv r; partials r.z and r.r
+// alpha from the partials of p.ap; x += alpha p, r -= alpha ap, z = dinv r;
+// partials r.z and r.r. The first element's loads do not wait for alpha.
 __global__ void __launch_bounds__(TPB) k_cg_update(double* __restrict__ x, double* __restrict__ r,
                                                    double* __restrict__ z,
                                                    const double* __restrict__ p,
                                                    const double* __restrict__ ap,
                                                    const double* __restrict__ dinv, int64_t n,
-                                                   const CgS* S, double* part) {
+                                                   const CgS* S, double* part, int np, int par) {
   if (S->done) return;
-  __shared__ double sh[TPB / 64];
-  const double alpha = S->alpha;
-  double rz = 0.0, rr = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    x[i] += alpha * p[i];
-    const double ri = r[i] - alpha * ap[i], zi = dinv[i] * ri;
-    r[i] = ri;
-    z[i] = zi;
-    rz += ri * zi;
-    rr += ri * ri;
+  __shared__ double sh2[TPB / 32];
+  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  double xi = 0.0, pi = 0.0, ri = 0.0, ai = 0.0, di = 0.0;
+  const auto fetch = [&] {
+    xi = x[i];
+    pi = p[i];
+    ri = r[i];
+    ai = ap[i];
+    di = dinv[i];
+  };
+  if (i < n) fetch();
+  double v = 0.0;
+  for (int q = threadIdx.x; q < np; q += TPB) v += part[CG_PAP + q];
+  double rr = 0.0;
+  block_sums(v, rr, sh2);
+  const double alpha = S->rz[par ^ 1] / v;
+  double rz = 0.0;
+  for (; i < n;) {
+    x[i] = xi + alpha * pi;
+    const double rn = ri - alpha * ai, zn = di * rn;
+    r[i] = rn;
+    z[i] = zn;
+    rz += rn * zn;
+    rr += rn * rn;
+    i += (int64_t)gridDim.x * blockDim.x;
+    if (i < n) fetch();
   }
-  const double t0 = block_reduce(rz, sh);
-  __syncthreads();
-  const double t1 = block_reduce(rr, sh);
+  __shared__ double sh3[TPB / 32];
+  block_sums(rz, rr, sh3);
   if (threadIdx.x == 0) {
-    part[blockIdx.x] = t0;
-    part[NBLK + blockIdx.x] = t1;
+    part[blockIdx.x] = rz;
+    part[CG_RR + blockIdx.x] = rr;
   }
 }
 
-__global__ void k_cg_beta(CgS* S, const double* part, int np) {
-  if (S->done) return;
-  __shared__ double sh[TPB / 64];
-  double a = 0.0, b = 0.0;
-  for (int i = threadIdx.x; i < np; i += blockDim.x) {
-    a += part[i];
-    b += part[NBLK + i];
-  }
-  const double rz = block_reduce(a, sh);
-  __syncthreads();
-  const double rr = block_reduce(b, sh);
-  if (threadIdx.x == 0) {
-    CgS s = *S;
-    s.beta = rz / s.rz;
-    s.rz = rz;
-    s.res2 = rr;
-    s.iter += 1;
-    if (rr <= s.rtol2 * s.bnorm2 || s.iter >= s.max_iters) s.done = 1;
-    *S = s;
-  }
-}
-
-// p = z + beta p
-__global__ void k_cg_dir(double* __restrict__ p, const double* __restrict__ z, int64_t n,
-                         const CgS* S) {
-  if (S->done) return;
-  const double beta = S->beta;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = z[i] + beta * p[i];
-}
-
-// Jacobi CG (krylov.rs:48-95: stop when |r| <= rtol |b|) with its scalars on
-// the device: five launches per iteration, one host read per CG_SEG iterations.
+// Jacobi CG (krylov.rs:48-95: stop when |r| <= rtol |b|) with its scalars on the device.
 namespace {
 
 // Device buffers of one CG run.
 struct CgWork {
-  double *r, *z, *p, *ap, *part;
+  double *r, *z, *p, *q, *ap, *part;  // p, q: the direction by parity
   CgS* S;
 };
 
@@ -3035,22 +3145,46 @@ KrylovStats cg_solve_ws(Ctx* ctx, const Csr& a, const double* dinv, const double
     ks.precond_residual = 0.0;
     return ks;
   }
-  const unsigned gr = red_grid(n), gs = spmv_grid(n);
+  const unsigned gr = std::min<unsigned>(red_grid(n), CG_RED), gs = std::min<unsigned>(spmv_grid(n), CG_ROWS);
+  static_assert(2 * sizeof(CgS) <= Ctx::kPinnedBytes, "CG states fit the pinned words");
+  CgS* host = static_cast<CgS*>(ctx->pinned);
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  struct Events {
+    hipEvent_t* e;
+    ~Events() {
+      for (int i = 0; i < 2; ++i)
+        if (e[i]) (void)hipEventDestroy(e[i]);
+    }
+  } owner{ev};
+  for (auto& e : ev) FEEC_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   k_cg_init<<<gr, TPB, 0, st>>>(b, dinv, n, x, w.r, w.z, w.p, w.part);
   k_cg_start<<<1, TPB, 0, st>>>(w.S, w.part, (int)gr, rtol, (long long)max_iters);
   CgS h{};
-  while (true) {
+  for (int seg = 0;; ++seg) {
     for (int it = 0; it < CG_SEG; ++it) {
-      k_cg_spmv<<<gs, TPB, 0, st>>>(a.row_ptr.p, a.col.p, a.val.p, n, w.p, w.ap, w.S, w.part);
-      k_cg_alpha<<<1, TPB, 0, st>>>(w.S, w.part, (int)gs);
-      k_cg_update<<<gr, TPB, 0, st>>>(x, w.r, w.z, w.p, w.ap, dinv, n, w.S, w.part);
-      k_cg_beta<<<1, TPB, 0, st>>>(w.S, w.part, (int)gr);
-      k_cg_dir<<<gr, TPB, 0, st>>>(w.p, w.z, n, w.S);
+      const int par = it & 1;
+      double* p0 = par ? w.q : w.p;
+      double* p1 = par ? w.p : w.q;
+      if (n <= CG_TWO_ROWS) {
+        k_cg_spmv<true><<<gs, TPB, 0, st>>>(a.row_ptr.p, a.col.p, a.val.p, n, w.z, p0, p1, w.ap, w.S, w.part,
+                                            (int)gr, par);
+      } else {
+        k_cg_dir<<<gr, TPB, 0, st>>>(w.z, p0, p1, n, w.S, w.part, (int)gr, par);
+        k_cg_spmv<false><<<gs, TPB, 0, st>>>(a.row_ptr.p, a.col.p, a.val.p, n, w.z, p0, p1, w.ap, w.S, w.part,
+                                             (int)gr, par);
+      }
+      k_cg_update<<<gr, TPB, 0, st>>>(x, w.r, w.z, p1, w.ap, dinv, n, w.S, w.part, (int)gs, par);
     }
     FEEC_HIP(hipGetLastError());
-    copy_to_host(ctx, &h, w.S, sizeof(h));
+    FEEC_HIP(hipMemcpyAsync(host + (seg & 1), w.S, sizeof(CgS), hipMemcpyDeviceToHost, st));
+    FEEC_HIP(hipEventRecord(ev[seg & 1], st));
+    if (seg == 0) continue;
+    FEEC_HIP(hipEventSynchronize(ev[(seg - 1) & 1]));
+    h = host[(seg - 1) & 1];
     if (h.done) break;
   }
+  // The segment in flight only returns, and its copy of the (final) state runs
+  // before anything later on the stream reuses the state or the pinned words.
   ks.iters = h.iter;
   ks.precond_residual = h.bnorm2 > 0.0 ? std::sqrt(h.res2 / h.bnorm2) : 0.0;
   ks.converged = h.bnorm2 == 0.0 || h.res2 <= h.rtol2 * h.bnorm2;
@@ -3060,13 +3194,13 @@ KrylovStats cg_solve_ws(Ctx* ctx, const Csr& a, const double* dinv, const double
 // ---------------------------------------------------------------------------
 // feec_csr_cg_noalloc's scratch: a file-scope device array, one copy per GPU
 // (each at its own address), held until the process ends. Layout, in doubles:
-// the CG scalars (padded to 256 B), 2 * NBLK partial sums, then seven vectors
-// of kNoAllocMaxRows: b, x (staging), the inverse diagonal, r, z, p, A p.
+// the CG scalars (padded to 256 B), 2 * NBLK partial sums, then eight vectors of
+// kNoAllocMaxRows: b, x (staging), the inverse diagonal, r, z, p (two), A p.
 // ---------------------------------------------------------------------------
 constexpr int64_t kNoAllocMaxRows = int64_t(1) << 18;
 constexpr int64_t kScalarDoubles = 32;
 static_assert(sizeof(CgS) <= kScalarDoubles * sizeof(double), "CG scalars fit their slot");
-constexpr int64_t kNoAllocDoubles = kScalarDoubles + 2 * NBLK + 7 * kNoAllocMaxRows;
+constexpr int64_t kNoAllocDoubles = kScalarDoubles + 2 * NBLK + 8 * kNoAllocMaxRows;
 static __device__ __align__(256) double scratch[kNoAllocDoubles];
 
 std::mutex g_scratch_mu;
@@ -3097,9 +3231,9 @@ void noalloc_scratch_init(int device) {
 KrylovStats cg_solve_device(Ctx* ctx, const Csr& a, const double* dinv, const double* b, double* x,
                             double rtol, int64_t max_iters) {
   const int64_t n = std::max<int64_t>(a.nrows, 1);
-  DBuf<double> r(ctx, n), z(ctx, n), p(ctx, n), ap(ctx, n), part(ctx, 2 * NBLK);
+  DBuf<double> r(ctx, n), z(ctx, n), p(ctx, n), q(ctx, n), ap(ctx, n), part(ctx, 2 * NBLK);
   DBuf<CgS> S(ctx, 1);
-  return cg_solve_ws(ctx, a, dinv, b, x, rtol, max_iters, CgWork{r.p, z.p, p.p, ap.p, part.p, S.p});
+  return cg_solve_ws(ctx, a, dinv, b, x, rtol, max_iters, CgWork{r.p, z.p, p.p, q.p, ap.p, part.p, S.p});
 }
 
 }  // namespace feec
@@ -3130,7 +3264,7 @@ feec_status feec_csr_cg_noalloc(feec_csr* a, const double* b, double* x, double 
     double* dx = v + kNoAllocMaxRows;
     double* dinv = v + 2 * kNoAllocMaxRows;
     const CgWork w{v + 3 * kNoAllocMaxRows, v + 4 * kNoAllocMaxRows, v + 5 * kNoAllocMaxRows,
-                   v + 6 * kNoAllocMaxRows, part, reinterpret_cast<CgS*>(base)};
+                   v + 6 * kNoAllocMaxRows, v + 7 * kNoAllocMaxRows, part, reinterpret_cast<CgS*>(base)};
     copy_to_device(ctx, db, b, n * 8);
     // Jacobi (precond.rs:53-123): the inverse diagonal, 1 where it is zero
     csr_diagonal(*a, dinv);

@@ -243,7 +243,7 @@ feec_status feec_csr_cg(feec_csr *a, const double *b, double *x, double rtol, in
  * capture, tight serving loops, harnesses that forbid hipMalloc). Same kernels,
  * same order, same results as feec_csr_cg; its vectors, partial sums and scalars
  * live in a file-scope device array set up by feec_ctx_create and held by each GPU
- * until the process ends (14.1 MiB: 262144 rows at most; larger a: FEEC_E_ARG).
+ * until the process ends (16.1 MiB: 262144 rows at most; larger a: FEEC_E_ARG).
  * Every call on one GPU shares that array, so calls that overlap on one GPU
  * (from several threads or contexts) race; serialize them. */
 feec_status feec_csr_cg_noalloc(feec_csr *a, const double *b, double *x, double rtol,

@@ -570,3 +570,27 @@ def test_harmonics_outside_a_ball(shape):
     assert rep.converged and len(p) == 1
     assert np.abs(u - u_o).max() <= 1e-8 * np.abs(u_o).max()
     assert abs(p[0] - p_o[0]) <= 1e-8 * max(abs(p_o[0]), 1.0)
+
+
+@pytest.mark.parametrize("d,n,k", [(1, 3, 0), (2, 5, 1), (2, 63, 0), (3, 9, 3), (3, 24, 1), (3, 35, 1)])
+def test_mass_cg_launch_forms(d, n, k):
+    """Jacobi CG on mass matrices from a few rows (one block, fewer rows than a
+    block's share) to beyond the two-launch form's 300,000 (3D 35^3 edges: 309 k):
+    the solution satisfies the system to the stop's rtol (the recurrence's
+    residual follows the true one to roundoff, 1e-14 of |b| per iteration), a
+    budget that ends the run is reported as such, and a zero right-hand side
+    takes no iteration."""
+    _, _, gcx, geo, _, _ = both(d, n, 0.05, seed=n)
+    A = fa.WhitneyComplex(geo).mass(k)
+    b = np.cos(np.arange(A.shape[0]) * 0.9)
+    x, rep = A.cg(b, rtol=1e-11)
+    assert rep.converged and rep.residual <= 1e-11
+    assert np.linalg.norm(A @ x - b) <= (1e-11 + 1e-14 * rep.iters) * np.linalg.norm(b)
+    x2, rep2 = A.cg(b, rtol=1e-11)
+    np.testing.assert_array_equal(x, x2)
+    if rep.iters > 1:
+        xs, short = A.cg(b, rtol=1e-11, max_iters=rep.iters - 1, raise_on_failure=False)
+        assert short.iters == rep.iters - 1 and not short.converged
+        assert short.residual > 1e-11
+    x0, zero = A.cg(0.0 * b, rtol=1e-11)
+    assert zero.iters == 0 and zero.converged and not x0.any()
