@@ -187,3 +187,20 @@ def test_topology_errors():
     with pytest.raises(fa.FeecError) as e:
         fa.Complex(2, np.array([[0, 1, 2], [0, 1, 3], [0, 1, 4]]), nverts=5)  # facet in 3 cells
     assert e.value.name == "FEEC_E_TOPOLOGY"
+
+
+@pytest.mark.parametrize("d,n,jitter", [(1, 1, 0.0), (1, 70, 0.1), (2, 1, 0.0), (2, 9, 0.0), (2, 13, 0.1), (3, 1, 0.0),
+                                        (3, 4, 0.0), (3, 5, 0.05), (4, 1, 0.0), (4, 2, 0.05)])
+@pytest.mark.parametrize("relative", [False, True])
+def test_hdif_gram_row_merge(d, n, jitter, relative):
+    """hdif_gram(k) = M_k + dif_both(k+1) merged row by row: on unjittered grids the
+    two patterns differ (each drops its own exact zeros), rows of one entry, empty
+    operands (k = d) and empty relative complexes among them; bit for bit the
+    oracle's sum."""
+    ocx, oL, gcx, geo, _, _ = both(d, n, jitter, seed=n)
+    oc, gc = o.WhitneyComplex(ocx, oL, relative=relative), fa.WhitneyComplex(geo, relative=relative)
+    for k in range(d + 1):
+        if oc.ndofs(k):
+            assert_csr_parity(gc.hdif_gram(k), oc.hdif_gram(k), what=f"hdif_gram({k})")
+        else:
+            assert gc.hdif_gram(k).nnz == 0
