@@ -514,14 +514,120 @@ __global__ void k_select_coo(const int64_t* row_ptr, const int32_t* col, int64_t
   }
 }
 
-// structural product: count terms per row of A
+// structural product: count terms per row of A, and the longest row
 __global__ void k_mul_count(const int64_t* arp, const int32_t* acol, const int64_t* brp,
-                            int64_t nrows, unsigned long long* cnt) {
-  int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (r >= nrows) return;
+                            int64_t nrows, unsigned long long* cnt, unsigned long long* longest) {
+  __shared__ unsigned long long top;
+  if (threadIdx.x == 0) top = 0;
+  __syncthreads();
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, r = t / ROW_LANES;
   unsigned long long c = 0;
-  for (int64_t p = arp[r]; p < arp[r + 1]; ++p) c += brp[acol[p] + 1] - brp[acol[p]];
-  cnt[r] = c;
+  if (r < nrows)
+    for (int64_t p = arp[r] + t % ROW_LANES; p < arp[r + 1]; p += ROW_LANES) c += brp[acol[p] + 1] - brp[acol[p]];
+#pragma unroll
+  for (int off = ROW_LANES / 2; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+  if (r <= nrows && t % ROW_LANES == 0) {
+    cnt[r] = c;  // 0 at nrows: the scan ends on the total
+    atomicMax(&top, c);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && top) atomicMax(longest, top);
+}
+
+// One row of the product per wavefront: its terms in the order of A's row go to
+// LDS under keys (column, place), a bitonic sort brings equal columns together
+// in that order, and each run's first lane adds it up from the left, as a
+// stable sort of all terms by (row, column) and a segmented sum would. The rows
+// come out at the terms' offsets; len[r] is what each kept. Rows of up to
+// MUL_ROW terms (a 4D mass row times the coboundary has about 400): against the
+// sort of all terms this reads and writes each one once instead of five times.
+constexpr int MUL_ROW = 512, MUL_BITS = 9;
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+__global__ void __launch_bounds__(TPB) k_mul_rows(const int64_t* arp, const int32_t* acol, const double* aval,
+                                                  const int64_t* brp, const int32_t* bcol, const double* bval,
+                                                  int64_t nrows, const int64_t* start, int32_t* tcol, double* tval,
+                                                  unsigned long long* len) {
+  __shared__ uint64_t keys_[TPB / 64][MUL_ROW];
+  __shared__ double vals_[TPB / 64][MUL_ROW];
+  uint64_t* keys = keys_[threadIdx.x / 64];
+  double* vals = vals_[threadIdx.x / 64];
+  const int lane = (int)(threadIdx.x & 63);
+  const int64_t r = blockIdx.x * (int64_t)(TPB / 64) + threadIdx.x / 64;
+  if (r > nrows) return;
+  if (r == nrows) {
+    if (lane == 0) len[r] = 0;
+    return;
+  }
+  const int64_t o = start[r];
+  const int m = (int)(start[r + 1] - o);
+  const int64_t p1 = arp[r + 1];
+  int at = 0;
+  for (int64_t p0 = arp[r]; p0 < p1; p0 += 64) {
+    const int64_t p = p0 + lane;
+    const bool here = p < p1;
+    const int32_t k = here ? acol[p] : 0;
+    const double av = here ? aval[p] : 0.0;
+    const int64_t q0 = here ? brp[k] : 0;
+    const int n = here ? (int)(brp[k + 1] - q0) : 0;
+    int before = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int up = __shfl_up(before, off, 64);
+      if (lane >= off) before += up;
+    }
+    const int all = __shfl(before, 63, 64);
+    int w = at + before - n;
+    for (int i = 0; i < n; ++i, ++w) {
+      keys[w] = (uint64_t)(uint32_t)bcol[q0 + i] << MUL_BITS | (uint64_t)w;
+      vals[w] = av * bval[q0 + i];
+    }
+    at += all;
+  }
+  int size = 1;
+  while (size < m) size <<= 1;
+  for (int i = m + lane; i < size; i += 64) keys[i] = ~uint64_t(0);
+  wave_lds_fence();
+  for (int k = 2; k <= size; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int h = lane; h < size / 2; h += 64) {
+        const int i = (h & (j - 1)) | (h & ~(j - 1)) << 1;  // the pair's lower place
+        const uint64_t a = keys[i], b = keys[i | j];
+        if ((a > b) == ((i & k) == 0)) {
+          keys[i] = b;
+          keys[i | j] = a;
+        }
+      }
+      wave_lds_fence();
+    }
+  int kept = 0;
+  for (int i0 = 0; i0 < m; i0 += 64) {
+    const int i = i0 + lane;
+    const uint64_t key = i < m ? keys[i] : 0;
+    const bool head = i < m && (i == 0 || (keys[i - 1] ^ key) >> MUL_BITS);
+    const uint64_t heads = __ballot(head);
+    if (head) {
+      double acc = vals[key & (MUL_ROW - 1)];
+      for (int j = i + 1; j < m && ((keys[j] ^ key) >> MUL_BITS) == 0; ++j) acc += vals[keys[j] & (MUL_ROW - 1)];
+      const int64_t w = o + kept + __popcll(heads & ((uint64_t(1) << lane) - 1));
+      tcol[w] = (int32_t)(key >> MUL_BITS);
+      tval[w] = acc;
+    }
+    kept += __popcll(heads);
+  }
+  if (lane == 0) len[r] = (unsigned long long)kept;
+}
+__global__ void k_mul_pack(const int64_t* start, const int32_t* tcol, const double* tval, int64_t nrows,
+                           const int64_t* orp, int32_t* ocol, double* oval) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, r = t / ROW_LANES;
+  if (r >= nrows) return;
+  const int64_t o = orp[r], n = orp[r + 1] - o, s = start[r];
+  for (int64_t i = t % ROW_LANES; i < n; i += ROW_LANES) {
+    ocol[o + i] = tcol[s + i];
+    oval[o + i] = tval[s + i];
+  }
 }
 
 // The terms of the product, row by row in the order of A's row: ROW_LANES lanes
@@ -686,28 +792,45 @@ void csr_select(const Csr& a, const int32_t* row_map, int64_t nrows, const int32
 void csr_mul(const Csr& a, const Csr& b, Csr& out) {
   Ctx* ctx = a.ctx;
   FEEC_REQUIRE(a.ncols == b.nrows, FEEC_E_ARG, "csr_mul shape mismatch");
-  DBuf<unsigned long long> cnt(ctx, std::max<int64_t>(a.nrows, 1));
-  DBuf<int64_t> start(ctx, std::max<int64_t>(a.nrows, 1));
-  if (a.nrows)
-    k_mul_count<<<grid_for(a.nrows), TPB, 0, ctx->stream>>>(a.row_ptr.p, a.col.p, b.row_ptr.p,
-                                                            a.nrows, cnt.p);
+  const int64_t n = a.nrows;
+  DBuf<unsigned long long> cnt(ctx, n + 1), longest(ctx, 1);
+  DBuf<int64_t> start(ctx, n + 1);
+  k_zero_counts<<<1, TPB, 0, ctx->stream>>>(longest.p, 1);
+  k_mul_count<<<row_grid(n + 1), TPB, 0, ctx->stream>>>(a.row_ptr.p, a.col.p, b.row_ptr.p, n, cnt.p, longest.p);
+  FEEC_HIP(hipGetLastError());
+  exclusive_scan_u64_to_i64<int64_t>(ctx, cnt.p, start.p, n + 1);
   int64_t total = 0;
-  if (a.nrows) {
-    exclusive_scan_u64_to_i64<int64_t>(ctx, cnt.p, start.p, a.nrows);
-    int64_t last_start = 0;
-    unsigned long long last_cnt = 0;
-    FEEC_HIP(hipMemcpyAsync(&last_start, start.p + a.nrows - 1, sizeof(int64_t),
-                            hipMemcpyDeviceToHost, ctx->stream));
-    FEEC_HIP(hipMemcpyAsync(&last_cnt, cnt.p + a.nrows - 1, sizeof(unsigned long long),
-                            hipMemcpyDeviceToHost, ctx->stream));
-    ctx->sync();
-    total = last_start + (int64_t)last_cnt;
-  }
+  unsigned long long most = 0;
+  FEEC_HIP(hipMemcpyAsync(&total, start.p + n, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
+  FEEC_HIP(hipMemcpyAsync(&most, longest.p, sizeof(most), hipMemcpyDeviceToHost, ctx->stream));
+  ctx->sync();
   FEEC_REQUIRE(total < (int64_t(1) << 31), FEEC_E_ARG, "product too large");
+  if (most <= MUL_ROW) {
+    DBuf<int32_t> tcol(ctx, std::max<int64_t>(total, 1));
+    DBuf<double> tval(ctx, std::max<int64_t>(total, 1));
+    k_mul_rows<<<(unsigned)(n / (TPB / 64) + 1), TPB, 0, ctx->stream>>>(a.row_ptr.p, a.col.p, a.val.p, b.row_ptr.p,
+                                                                       b.col.p, b.val.p, n, start.p, tcol.p, tval.p,
+                                                                       cnt.p);
+    FEEC_HIP(hipGetLastError());
+    out.ctx = ctx;
+    out.nrows = n;
+    out.ncols = b.ncols;
+    out.row_ptr.alloc(ctx, n + 1);
+    exclusive_scan_u64_to_i64<int64_t>(ctx, cnt.p, out.row_ptr.p, n + 1);
+    copy_to_host(ctx, &out.nnz, out.row_ptr.p + n, sizeof(int64_t));
+    out.col.alloc(ctx, out.nnz);
+    out.val.alloc(ctx, out.nnz);
+    if (n)
+      k_mul_pack<<<row_grid(n), TPB, 0, ctx->stream>>>(start.p, tcol.p, tval.p, n, out.row_ptr.p, out.col.p,
+                                                       out.val.p);
+    FEEC_HIP(hipGetLastError());
+    ctx->sync();
+    return;
+  }
   DBuf<int32_t> rows(ctx, total), cols(ctx, total);
   DBuf<uint32_t> srcs(ctx, total);
   DBuf<double> vals(ctx, total);
-  if (a.nrows)
+  if (n)
     k_mul_terms<<<row_grid(a.nrows), TPB, 0, ctx->stream>>>(
         a.row_ptr.p, a.col.p, a.val.p, b.row_ptr.p, b.col.p, b.val.p, a.nrows, start.p, rows.p,
         cols.p, srcs.p, vals.p);

@@ -204,3 +204,25 @@ def test_hdif_gram_row_merge(d, n, jitter, relative):
             assert_csr_parity(gc.hdif_gram(k), oc.hdif_gram(k), what=f"hdif_gram({k})")
         else:
             assert gc.hdif_gram(k).nnz == 0
+
+
+@pytest.mark.parametrize("m", [3, 84, 85, 86, 200])
+def test_dirac_product_rows(m):
+    """U_1 = M_1 D_0 on m tets around one edge: that edge's mass row has 3m + 1
+    entries, so its product row (6m + 2 terms) lies below, at the last multiple
+    below, and beyond the 512 terms that a wavefront sorts; bit for bit the
+    oracle's block operator either way."""
+    t = 2.0 * np.pi * np.arange(m) / m
+    coords = np.concatenate([[[0.0, 0.0, -1.0], [0.1, 0.05, 1.0]],
+                             np.stack([np.cos(t), np.sin(t), 0.1 * np.cos(3 * t)], 1)])
+    ring = 2 + np.arange(m)
+    cells = np.stack([np.zeros(m, int), np.ones(m, int), ring, np.roll(ring, -1)], 1)
+    ocx = o.Complex(3, cells)
+    gcx = fa.Complex(3, cells, nverts=len(coords))
+    geo = fa.MeshLengthsSq.from_coords(gcx, coords)
+    oc = o.WhitneyComplex(ocx, ocx.lengths_from_coords(coords))
+    offsets, mass, op = o.hodge_dirac(oc, -1.0)
+    hd = fa.HodgeDirac.assemble(fa.WhitneyComplex(geo))
+    np.testing.assert_array_equal(hd.offsets, offsets)
+    assert_csr_parity(hd.mass_block, mass, what="mass block")
+    assert_csr_parity(hd.op, op, what="operator")
