@@ -75,7 +75,7 @@ namespace {
 constexpr int TPB = 256;
 constexpr int NBLK = 4096;
 constexpr int MAXNV = 16;               // slots of one multi-right-hand-side cycle
-constexpr int MAXC = 8;                 // values per entry of a transfer matrix
+constexpr int MAXC = 10;                // values per entry of a transfer matrix
 constexpr int64_t kCoarseMax = 200;     // largest level solved directly (unknowns)
 constexpr int64_t kDenseMaxBox = 1024;  // largest coarsest box
 constexpr double kOmega = 2.0 / 3.0;
@@ -1009,91 +1009,197 @@ __global__ void __launch_bounds__(TPB) k_st_galerkin(const double* __restrict__ 
 // ---------------------------------------------------------------------------
 // HX transfers between the KKT vector and the level-0 slots
 // ---------------------------------------------------------------------------
-// y[(slot0 + v) * ny + row] = sum_p val[p * C + v] x[col[p]] for v < C; LPR
-// lanes share a row (entries strided over them, summed by shuffles).
-template <class TX, class TP, int LPR>
-__global__ void __launch_bounds__(TPB) k_hx_gather(const int64_t* __restrict__ rp,
-                                                   const int32_t* __restrict__ col,
-                                                   const TP* __restrict__ val, int C,
-                                                   const TX* __restrict__ x, TP* __restrict__ y, int64_t ny,
-                                                   int slot0, int64_t nrows, const MinresS* S) {
-  if (skip(S)) return;
-  const int64_t gid = xcd_block() * (int64_t)blockDim.x + threadIdx.x;
+// One launch gathers the block residuals into the slots and one scatters the
+// cycle's result back, whatever the blocks: each is a list of jobs with blocks
+// of their own (a multiple of the 8 XCDs each, contiguous rows an XCD), so the
+// small ones cost no launch and run beside the large ones.
+constexpr int MAXJOBS = 4;
+inline unsigned job_blocks(int64_t threads) { return (grid_for(threads) + 7) / 8 * 8; }
+// The job of this block and its block within the job, XCD by XCD.
+template <class J>
+__device__ __forceinline__ int find_job(const J* jobs, int n, unsigned& blk) {
+  unsigned b = blockIdx.x;
+  int q = 0;
+  while (q + 1 < n && b >= jobs[q].blocks) b -= jobs[q++].blocks;
+  blk = (b % 8) * (jobs[q].blocks / 8) + b / 8;
+  return q;
+}
+
+// y[v * ny + row] = sum_p val[p * C + v] x[col[p]] for v < C; lpr lanes (1 or 4)
+// share a row, entries strided over them, summed by shuffles.
+template <class TX, class TP>
+struct GatherJob {
+  const int64_t* rp;
+  const int32_t* col;
+  const TP* val;
+  const TX* x;
+  TP* y;
+  int64_t ny, nrows;
+  int C, lpr;
+  unsigned blocks;
+};
+template <class TX, class TP>
+struct GatherJobs {
+  GatherJob<TX, TP> j[MAXJOBS];
+  int n;
+};
+// C values of entry p added into acc with weight x; the values of 4 and 6 are
+// read 4 and 2 at a time (their places are so aligned).
+template <class TP, int C>
+__device__ __forceinline__ void add_entry(const TP* __restrict__ val, int64_t p, TP x, TP (&acc)[MAXC]) {
+  constexpr int W = C % 4 == 0 ? 4 : C % 2 == 0 ? 2 : 1;
+  typedef TP vec __attribute__((ext_vector_type(W)));
+#pragma unroll
+  for (int w = 0; w < C / W; ++w) {
+    if constexpr (W == 1) {
+      acc[w] += val[p * C + w] * x;
+    } else {
+      const vec q = *reinterpret_cast<const vec*>(val + p * C + w * W);
+#pragma unroll
+      for (int i = 0; i < W; ++i) acc[w * W + i] += q[i] * x;
+    }
+  }
+}
+template <class TX, class TP, int LPR, int C>
+__device__ __forceinline__ void gather_rows(const GatherJob<TX, TP>& g, unsigned blk) {
+  const int64_t gid = blk * (int64_t)TPB + threadIdx.x;
   const int64_t row = gid / LPR;
   const int lane = (int)(gid % LPR);
   TP acc[MAXC];
 #pragma unroll
-  for (int v = 0; v < MAXC; ++v) acc[v] = TP(0);
-  if (row < nrows) {
-    for (int64_t p = rp[row] + lane; p < rp[row + 1]; p += LPR) {
-      const TP xv = (TP)x[col[p]];
-#pragma unroll
-      for (int v = 0; v < MAXC; ++v)
-        if (v < C) acc[v] += val[p * C + v] * xv;
-    }
+  for (int v = 0; v < C; ++v) acc[v] = TP(0);
+  if (row < g.nrows) {
+    const int64_t e = g.rp[row + 1];
+    for (int64_t p = g.rp[row] + lane; p < e; p += LPR) add_entry<TP, C>(g.val, p, (TP)g.x[g.col[p]], acc);
   }
-  if (LPR > 1) {
 #pragma unroll
-    for (int v = 0; v < MAXC; ++v) {
-      TP t = acc[v];
+  for (int v = 0; v < C; ++v) {
+    TP t = acc[v];
 #pragma unroll
-      for (int off = LPR / 2; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-      acc[v] = t;
-    }
+    for (int off = LPR / 2; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+    if (row < g.nrows && lane == 0) g.y[v * g.ny + row] = t;
   }
-  if (row < nrows && lane == 0)
-    for (int v = 0; v < C; ++v) y[(slot0 + v) * ny + row] = acc[v];
 }
-
-// y[row] = (a ? a[row] b[row] : add ? y[row] : 0)
-//          + sum_p sum_v val[p * C + v] X(col[p], v),
-// X(c, v) = x0[(slot0 + v) * nx + c], except X(c, 0) = x0[..] + dl[c] r0[..]
-// when `grad` (the grade-0 term S_0 t + V t of the gradient correction).
-template <class TP, class TA, class TB>
-__global__ void __launch_bounds__(TPB) k_hx_out(const int64_t* __restrict__ rp, const int32_t* __restrict__ col,
-                                                const TP* __restrict__ val, int C, int grad,
-                                                const TP* __restrict__ x0, const TP* __restrict__ r0,
-                                                const TP* __restrict__ dl, int64_t nx, int slot0,
-                                                const TA* __restrict__ a, const TB* __restrict__ b,
-                                                TP* __restrict__ y, int64_t nrows, int add, const MinresS* S) {
+template <class TX, class TP, int LPR>
+__device__ __forceinline__ void gather_by_width(const GatherJob<TX, TP>& g, unsigned blk) {
+  switch (g.C) {
+    case 1: gather_rows<TX, TP, LPR, 1>(g, blk); break;
+    case 2: gather_rows<TX, TP, LPR, 2>(g, blk); break;
+    case 3: gather_rows<TX, TP, LPR, 3>(g, blk); break;
+    case 4: gather_rows<TX, TP, LPR, 4>(g, blk); break;
+    case 5: gather_rows<TX, TP, LPR, 5>(g, blk); break;
+    case 6: gather_rows<TX, TP, LPR, 6>(g, blk); break;
+    default: gather_rows<TX, TP, LPR, 10>(g, blk); break;
+  }
+}
+inline bool gather_width(int C) { return (C >= 1 && C <= 6) || C == 10; }
+template <class TX, class TP>
+__global__ void __launch_bounds__(TPB) k_hx_gather(GatherJobs<TX, TP> jobs, const MinresS* S) {
   if (skip(S)) return;
-  const int64_t i = xcd_block() * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= nrows) return;
-  TP acc = a ? (TP)a[i] * (TP)b[i] : (add ? y[i] : TP(0));
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p) {
-    const int64_t base = slot0 * nx + col[p];
-    TP x = x0[base];
-    if (grad) x += dl[col[p]] * r0[base];
-    acc += val[p * C] * x;
-    for (int v = 1; v < C; ++v) acc += val[p * C + v] * x0[base + v * nx];
-  }
-  y[i] = acc;
+  unsigned blk;
+  const GatherJob<TX, TP>& g = jobs.j[find_job(jobs.j, jobs.n, blk)];
+  if (g.lpr == 4)
+    gather_by_width<TX, TP, 4>(g, blk);
+  else
+    gather_by_width<TX, TP, 1>(g, blk);
 }
 
-// The grade-1 block's scatter without a matrix: row e is the edge (v0, v1),
-// v0 < v1 (box vertices), D_0 has -1 at v0 and +1 at v1 and Pi_1 the same D
+// B r on the rows of a block: v = s r + sum_p sum_c val[p * C + c] X(col[p], c)
+// [+ sum_q dval[q] sl[dcol[q]] t[dcol[q]]], X(c, i) = x0[(slot0 + i) * nx + c],
+// except X(c, 0) = x0[..] + dl[c] r0[..] when `grad` (the grade-0 term
+// S_0 t + V t of the gradient correction); the bracket is D_1 S_1 D_1^T r of a
+// grade-2 block. An edge block without a matrix (ev) has row e = (v0, v1),
+// v0 < v1 (box vertices), D_0 with -1 at v0 and +1 at v1 and Pi_1 with the same D
 // values eh = (x(v1) - x(v0)) / 2 at both ends:
-//   z[e] = s[e] r[e] + (G(v1) - G(v0)) + sum_c eh[e, c] (X_c(v0) + X_c(v1)),
+//   v = s r + (G(v1) - G(v0)) + sum_c eh[e, c] (X_c(v0) + X_c(v1)),
 // G(v) = x0[slot0, v] + dl[v] r0[slot0, v] and X_c(v) = x0[slot0 + 1 + c, v].
 // Vertices that are not unknowns hold zeros in every slot, so both ends are
-// always read.
-template <class TP, class TB, int D>
-__global__ void __launch_bounds__(TPB) k_hx_out_edge(const int32_t* __restrict__ ev, const TP* __restrict__ eh,
-                                                     const TP* __restrict__ x0, const TP* __restrict__ r0,
-                                                     const TP* __restrict__ dl, int64_t nx, int slot0,
-                                                     const TP* __restrict__ s, const TB* __restrict__ r,
-                                                     TP* __restrict__ z, int64_t nrows, const MinresS* S) {
+// always read. MODE: what becomes of v, the block's row of the preconditioned
+// residual:
+//   0: zt = v
+//   1: the Chebyshev start: res = v, d = v / theta, z = 0
+//   2: step k: res -= v, z += d, d = rho_{k+1} rho_k d + 2 rho_{k+1} / delta res
+template <class TP, class TB>
+struct OutJob {
+  const int64_t* rp;
+  const int32_t* col;
+  const TP* val;
+  const int64_t* drp;
+  const int32_t* dcol;
+  const TP* dval;
+  const TP* sl;
+  const TP* t;
+  const int32_t* ev;
+  const TP* eh;
+  const TP* s;
+  const TB* r;
+  int64_t off, nrows;
+  int C, grad, slot0, block;  // block: 0 sigma, 1 u (the Chebyshev coefficients)
+  unsigned blocks;
+};
+template <class TP, class TB>
+struct OutJobs {
+  OutJob<TP, TB> j[MAXJOBS];
+  int n;
+};
+template <class TP>
+struct ChebVecs {
+  TP *zt, *res, *d, *z;
+  const double* coef;
+  int k;
+};
+template <class TP, class TB, int D, int MODE>
+__global__ void __launch_bounds__(TPB) k_hx_out(OutJobs<TP, TB> jobs, const TP* __restrict__ x0,
+                                                const TP* __restrict__ r0, const TP* __restrict__ dl, int64_t nx,
+                                                ChebVecs<TP> c, const MinresS* S) {
   if (skip(S)) return;
-  const int64_t e = xcd_block() * (int64_t)blockDim.x + threadIdx.x;
-  if (e >= nrows) return;
-  const int v0 = ev[2 * e], v1 = ev[2 * e + 1];
-  const TP* a = x0 + slot0 * nx + v0;
-  const TP* b = x0 + slot0 * nx + v1;
-  TP acc = s[e] * (TP)r[e];
-  acc += (b[0] + dl[v1] * r0[slot0 * nx + v1]) - (a[0] + dl[v0] * r0[slot0 * nx + v0]);
+  unsigned blk;
+  const OutJob<TP, TB>& g = jobs.j[find_job(jobs.j, jobs.n, blk)];
+  const int64_t i = blk * (int64_t)TPB + threadIdx.x;
+  if (i >= g.nrows) return;
+  const int64_t row = g.off + i;
+  TP res = TP(0), di = TP(0), zi = TP(0);
+  if (MODE == 2) {
+    res = c.res[row];
+    di = c.d[row];
+    zi = c.z[row];
+  }
+  TP acc = g.s[i] * (TP)g.r[i];
+  if (g.ev) {
+    const int v0 = g.ev[2 * i], v1 = g.ev[2 * i + 1];
+    const TP* a = x0 + g.slot0 * nx + v0;
+    const TP* b = x0 + g.slot0 * nx + v1;
+    acc += (b[0] + dl[v1] * r0[g.slot0 * nx + v1]) - (a[0] + dl[v0] * r0[g.slot0 * nx + v0]);
 #pragma unroll
-  for (int c = 0; c < D; ++c) acc += eh[e * D + c] * (a[(1 + c) * nx] + b[(1 + c) * nx]);
-  z[e] = acc;
+    for (int q = 0; q < D; ++q) acc += g.eh[i * D + q] * (a[(1 + q) * nx] + b[(1 + q) * nx]);
+  } else {
+    const int64_t e = g.rp[i + 1];
+    for (int64_t p = g.rp[i]; p < e; ++p) {
+      const int64_t base = g.slot0 * nx + g.col[p];
+      TP x = x0[base];
+      if (g.grad) x += dl[g.col[p]] * r0[base];
+      acc += g.val[p * g.C] * x;
+      for (int v = 1; v < g.C; ++v) acc += g.val[p * g.C + v] * x0[base + v * nx];
+    }
+    if (g.drp)
+      for (int64_t p = g.drp[i]; p < g.drp[i + 1]; ++p) {
+        const int32_t q = g.dcol[p];
+        acc += g.dval[p] * (g.sl[q] * g.t[q]);
+      }
+  }
+  if (MODE == 0) {
+    c.zt[row] = acc;
+  } else if (MODE == 1) {
+    c.res[row] = acc;
+    c.d[row] = acc * (TP)c.coef[g.block];
+    c.z[row] = TP(0);
+  } else {
+    const double* q = c.coef + 2 + 3 * c.k;
+    res -= acc;
+    c.res[row] = res;
+    c.z[row] = zi + di;
+    c.d[row] = (TP)q[0] * di + (TP)q[1 + g.block] * res;
+  }
 }
 
 __device__ __forceinline__ double dev_block_sum(double v, double* sh) {
@@ -1222,38 +1328,6 @@ __global__ void __launch_bounds__(TPB) k_pc_spmv32(const int64_t* __restrict__ r
 #pragma unroll
   for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
   if (row < nrows && lane == 0) y[row] = acc;
-}
-
-// res = zt, d = res / theta, z = 0
-template <class TP>
-__global__ void __launch_bounds__(TPB) k_hxc_first(const TP* __restrict__ zt, TP* __restrict__ res,
-                                                   TP* __restrict__ d, TP* __restrict__ z, int64_t n,
-                                                   int64_t split, const double* __restrict__ coef,
-                                                   const MinresS* S) {
-  if (skip(S)) return;
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const TP r = zt[i];
-  res[i] = r;
-  d[i] = r * (TP)coef[i < split ? 0 : 1];
-  z[i] = TP(0);
-}
-
-// step k: res -= zt, z += d, d = rho_{k+1} rho_k d + 2 rho_{k+1}/delta res
-template <class TP>
-__global__ void __launch_bounds__(TPB) k_hxc_step(const TP* __restrict__ zt, TP* __restrict__ res,
-                                                  TP* __restrict__ d, TP* __restrict__ z, int64_t n,
-                                                  int64_t split, const double* __restrict__ coef, int k,
-                                                  const MinresS* S) {
-  if (skip(S)) return;
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double* c = coef + 2 + 3 * k;
-  const TP r = res[i] - zt[i];
-  const TP di = d[i];
-  res[i] = r;
-  z[i] += di;
-  d[i] = (TP)c[0] * di + (TP)c[i < split ? 1 : 2] * r;
 }
 
 // out = z + d on the preconditioned rows, r on the border rows, and the
@@ -1531,18 +1605,18 @@ struct XCsr {
 struct HxBlock {
   int j = -1;  // grade of the block
   int64_t off = 0, n = 0;
-  // into the level-0 slots from the block's residual: j = 0 the nodal DOF
-  // map, j = 1 [D_0^T | Pi_1^T] (the gradient slot, then the Pi slots), j = 2 Pi_2^T
+  // into the level-0 slots from the block's residual: j = 0 the nodal DOF map,
+  // j = 1 [D_0^T | Pi_1^T] (the gradient slot, then the Pi slots), j = 2
+  // [Pi_2^T | (D_1 Pi_1)^T] (the Pi_2 slots, then those of the curl part)
   XCsr g_main;
   int slot_main = 0;
-  // back onto the block: j = 0 the map, j = 1 [D_0 | Pi_1] (gradient), j = 2 Pi_2
+  // back onto the block: j = 0 the map, j = 1 [D_0 | Pi_1] (gradient), j = 2 [Pi_2 | D_1 Pi_1]
   XCsr o_main;
-  // j = 2 only: t = D_1^T r, Pi_1^T t into the slots, u = S_1 t + Pi_1 (V ..), z += D_1 u
-  XCsr g_t, g_tl, o_ul, o_d;
-  int slot_tl = 0;
-  DBuf<double> sl, t64, u64;  // sl = S_1 on the grade-1 DOFs
-  DBuf<float> sl32, t32, u32;
-  // j = 1: the scatter without a matrix (k_hx_out_edge) when D_0's signs follow
+  // j = 2 only: t = D_1^T r, z += D_1 (S_1 t)
+  XCsr g_t, o_d;
+  DBuf<double> sl, t64;  // sl = S_1 on the grade-1 DOFs
+  DBuf<float> sl32, t32;
+  // j = 1: the scatter without a matrix (k_hx_out's ev) when D_0's signs follow
   // the sorted ends: the ends per row and the Pi_1 values
   bool edge_free = false;
   DBuf<int32_t> ev;
@@ -1760,6 +1834,25 @@ __global__ void k_gather_entries(const int64_t* seg, const uint32_t* src, const 
   out[q] = in[(int64_t)src[seg[e]] * C + (q - e * C)];
 }
 
+// (D Pi)'s values on the pattern of `rp`, `col` (which holds every column of the
+// product's row): entry (r, v) takes sum_q D(r, q) Pi(q, v), C values.
+__global__ void k_compose(const int64_t* rp, const int32_t* col, int64_t nrows, const int64_t* drp,
+                          const int32_t* dcol, const double* dval, const int64_t* prp, const int32_t* pcol,
+                          const double* pval, int C, double* out) {
+  const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (r >= nrows) return;
+  for (int64_t p = rp[r]; p < rp[r + 1]; ++p)
+    for (int v = 0; v < C; ++v) {
+      double acc = 0.0;
+      for (int64_t q = drp[r]; q < drp[r + 1]; ++q) {
+        const int32_t e = dcol[q];
+        for (int64_t s = prp[e]; s < prp[e + 1]; ++s)
+          if (pcol[s] == col[p]) acc += dval[q] * pval[s * C + v];
+      }
+      out[p * C + v] = acc;
+    }
+}
+
 // [a | b] on one pattern: a's C_a values, then b's C_b values, per entry;
 // bad[0] set when the patterns differ
 __global__ void k_interleave(const int64_t* arp, const int32_t* acol, const double* av, int ca,
@@ -1923,6 +2016,29 @@ void interleave_dev(Ctx* ctx, const XCsr& a, const XCsr& b, XCsr& out, int* bad)
     k_interleave<<<grid_for(am.nrows), TPB, 0, ctx->stream>>>(am.row_ptr.p, am.col.p, am.val.p, a.C,
                                                                b.m.row_ptr.p, b.m.col.p, b.m.val.p, b.C,
                                                                am.nrows, c.val.p, bad);
+  }
+  FEEC_HIP(hipGetLastError());
+  finish_x(ctx, out);
+}
+
+// D Pi on the pattern of `like` (which covers the product's).
+void compose_dev(Ctx* ctx, const XCsr& D, const XCsr& Pi, const XCsr& like, XCsr& out) {
+  const Csr& lm = like.m;
+  Csr& c = out.m;
+  c.ctx = ctx;
+  c.nrows = lm.nrows;
+  c.ncols = lm.ncols;
+  c.nnz = lm.nnz;
+  out.C = Pi.C;
+  c.row_ptr.alloc(ctx, lm.nrows + 1);
+  c.col.alloc(ctx, std::max<int64_t>(c.nnz, 1));
+  c.val.alloc(ctx, std::max<int64_t>(c.nnz * out.C, 1));
+  FEEC_HIP(hipMemcpyAsync(c.row_ptr.p, lm.row_ptr.p, (lm.nrows + 1) * 8, hipMemcpyDeviceToDevice, ctx->stream));
+  if (lm.nnz) {
+    FEEC_HIP(hipMemcpyAsync(c.col.p, lm.col.p, lm.nnz * 4, hipMemcpyDeviceToDevice, ctx->stream));
+    k_compose<<<grid_for(lm.nrows), TPB, 0, ctx->stream>>>(lm.row_ptr.p, lm.col.p, lm.nrows, D.m.row_ptr.p,
+                                                           D.m.col.p, D.m.val.p, Pi.m.row_ptr.p, Pi.m.col.p,
+                                                           Pi.m.val.p, out.C, c.val.p);
   }
   FEEC_HIP(hipGetLastError());
   finish_x(ctx, out);
@@ -2384,27 +2500,29 @@ Hx* hx_create(Geom& g, int bc, int k, const KktSystem& s, int sweeps, int cheb_m
       DBuf<int32_t> order_j, order_l;
       row_order(m, map_j, 2, b.n, order_j);
       row_order(m, map_l, 1, nl, order_l);
+      XCsr Pi, Pl, DPl;
       coboundary_dev(m, 2, map_j, b.n, map_l, nl, b.o_d);
-      vector_nodal_dev(m, X, 2, order_j.p, live_col_dev, b.n, nb0, b.o_main);
-      vector_nodal_dev(m, X, 1, order_l.p, live_col_dev, nl, nb0, b.o_ul);
+      vector_nodal_dev(m, X, 2, order_j.p, live_col_dev, b.n, nb0, Pi);
+      vector_nodal_dev(m, X, 1, order_l.p, live_col_dev, nl, nb0, Pl);
+      // the curl part's copies enter and leave through D_1 Pi_1, on Pi_2's pattern
+      // (a face's live vertices hold those of its edges)
+      compose_dev(ctx, b.o_d, Pl, Pi, DPl);
+      DBuf<int> bad(ctx, 1);
+      k_zero_i32<<<1, 64, 0, ctx->stream>>>(bad.p, 1);
+      interleave_dev(ctx, Pi, DPl, b.o_main, bad.p);
       transpose_dev(ctx, b.o_d, b.g_t);
-      transpose_dev(ctx, b.o_ul, b.g_tl);
       transpose_dev(ctx, b.o_main, b.g_main);
       b.slot_main = slot;
       slot += b.o_main.C;
-      b.slot_tl = slot;
-      slot += b.o_ul.C;
       b.t64.alloc(ctx, std::max<int64_t>(nl, 1));
-      b.u64.alloc(ctx, std::max<int64_t>(nl, 1));
       b.t32.alloc(ctx, std::max<int64_t>(nl, 1));
-      b.u32.alloc(ctx, std::max<int64_t>(nl, 1));
     }
     h->blocks.push_back(std::move(b));
   }
   if (slot > MAXNV) return no("too many auxiliary copies for one cycle");
   for (const auto& b : h->blocks)
-    for (const XCsr* x : {&b.g_main, &b.o_main, &b.g_t, &b.g_tl, &b.o_ul, &b.o_d})
-      if (x->C > MAXC) return no("too many components per transfer entry");
+    for (const XCsr* x : {&b.g_main, &b.g_t})
+      if (x->m.nnz && !gather_width(x->C)) return no("too many components per transfer entry");
   h->nv = slot;
   h->tail32 = tail_start<float>(*h);
   h->tail64 = tail_start<double>(*h);
@@ -2435,7 +2553,7 @@ Hx* hx_create(Geom& g, int bc, int k, const KktSystem& s, int sweeps, int cheb_m
     }
   }
   // work estimate of one application in FP32
-  int64_t bytes = 0, launches = 1;
+  int64_t bytes = 0, launches = 0;
   for (size_t i = 0; i < h->L.size(); ++i) {
     const MgLevel& l = h->L[i];
     const int64_t nbv = (int64_t)l.box.nb * h->nv;
@@ -2448,14 +2566,12 @@ Hx* hx_create(Geom& g, int bc, int k, const KktSystem& s, int sweeps, int cheb_m
     }
   }
   for (const auto& b : h->blocks)
-    for (const XCsr* x : {&b.g_main, &b.o_main, &b.g_t, &b.g_tl, &b.o_ul, &b.o_d})
-      if (x->m.nnz) {
-        bytes += x->m.nnz * 4 * (1 + x->C) + x->m.nrows * 8;
-        launches += 1;
-      }
+    for (const XCsr* x : {&b.g_main, &b.o_main, &b.g_t, &b.o_d})
+      if (x->m.nnz) bytes += x->m.nnz * 4 * (1 + x->C) + x->m.nrows * 8;
+  launches += 2;
   if (h->cheb_m > 1) {
     bytes = bytes * h->cheb_m + (h->cheb_m - 1) * (s.P.nnz * (h->P_col16.p ? 6 : 8) + h->n * 28) + h->n * 12;
-    launches = launches * h->cheb_m + 2 * (h->cheb_m - 1) + 2;
+    launches = launches * h->cheb_m + (h->cheb_m - 1) + 1;
   }
   h->bytes32 = bytes;
   h->launches = launches;
@@ -2525,7 +2641,6 @@ struct Sel<double> {
   static const double* v(const XCsr& x) { return x.m.val.p; }
   static const double* sl(const HxBlock& b) { return b.sl.p; }
   static double* t(HxBlock& b) { return b.t64.p; }
-  static double* u(HxBlock& b) { return b.u64.p; }
   static const double* eh(const HxBlock& b) { return b.eh64.p; }
   static double* res(Hx& h) { return h.res64.p; }
   static double* d(Hx& h) { return h.d64.p; }
@@ -2546,7 +2661,6 @@ struct Sel<float> {
   static const float* v(const XCsr& x) { return x.v32.p; }
   static const float* sl(const HxBlock& b) { return b.sl32.p; }
   static float* t(HxBlock& b) { return b.t32.p; }
-  static float* u(HxBlock& b) { return b.u32.p; }
   static const float* eh(const HxBlock& b) { return b.eh32.p; }
   static float* res(Hx& h) { return h.res32.p; }
   static float* d(Hx& h) { return h.d32.p; }
@@ -2712,58 +2826,63 @@ TP* vcycle(Enq& q, Hx& h, size_t i, const MinresS* S) {
   return x;
 }
 
-template <class TX, class TP>
-void gather(Enq& q, const XCsr& g, const TX* x, TP* y, int64_t ny, int slot0, const MinresS* S) {
-  using X = Sel<TP>;
-  const int64_t nr = g.m.nrows;
-  if (g.avg_row >= 6.0)
-    q(k_hx_gather<TX, TP, 4>, grid_for(nr * 4), TPB, g.m.row_ptr.p, g.m.col.p, X::v(g), g.C, x, y, ny, slot0,
-      nr, S);
-  else
-    q(k_hx_gather<TX, TP, 1>, grid_for(nr), TPB, g.m.row_ptr.p, g.m.col.p, X::v(g), g.C, x, y, ny, slot0, nr,
-      S);
-}
-
-// zt = B r on the preconditioned rows (r of length n at least).
-template <class TIN, class TP, int D>
-void hx_core_d(Enq& q, Hx& h, const TIN* r, const MinresS* S) {
+// B r on the preconditioned rows (r of length n at least): into zt (MODE 0), or
+// straight into the Chebyshev vectors (k_hx_out).
+template <class TIN, class TP, int D, int MODE = 0>
+void hx_core_d(Enq& q, Hx& h, const TIN* r, const MinresS* S, int k = 0) {
   using X = Sel<TP>;
   MgLevel& l0 = h.L[0];
   TP* slots = X::r(l0);
-  TP* zt = X::zt(h);
   const int64_t nx = l0.box.nb;
-  for (HxBlock& b : h.blocks) {
-    const TIN* rb = r + b.off;
-    if (b.j == 2) {
-      gather<TIN, TP>(q, b.g_t, rb, X::t(b), nx, 0, S);
-      gather<TP, TP>(q, b.g_tl, (const TP*)X::t(b), slots, nx, b.slot_tl, S);
-    }
-    gather<TIN, TP>(q, b.g_main, rb, slots, nx, b.slot_main, S);
+  GatherJobs<TIN, TP> in{};
+  unsigned blocks = 0;
+  const auto gather = [&](const XCsr& g, const TIN* x, TP* y) {
+    GatherJob<TIN, TP>& j = in.j[in.n++];
+    j = {g.m.row_ptr.p, g.m.col.p, X::v(g), x, y, nx, g.m.nrows, g.C, g.avg_row >= 6.0 ? 4 : 1, 0};
+    j.blocks = job_blocks(j.nrows * j.lpr);
+    blocks += j.blocks;
+  };
+  // the largest operator's blocks first
+  for (size_t i = h.blocks.size(); i-- > 0;) {
+    HxBlock& b = h.blocks[i];
+    gather(b.g_main, r + b.off, slots + b.slot_main * nx);
+    if (b.j == 2) gather(b.g_t, r + b.off, X::t(b));
   }
+  q(k_hx_gather<TIN, TP>, blocks, TPB, in, S);
   const TP* xs = vcycle<TP, D>(q, h, 0, S);
-  for (HxBlock& b : h.blocks) {
-    TP* zb = zt + b.off;
-    const TIN* rb = r + b.off;
-    const TP* sb = X::s(h) + b.off;
-    const XCsr& om = b.o_main;
+  OutJobs<TP, TIN> out{};
+  blocks = 0;
+  for (size_t i = h.blocks.size(); i-- > 0;) {
+    HxBlock& b = h.blocks[i];
+    OutJob<TP, TIN>& j = out.j[out.n++];
+    j.s = X::s(h) + b.off;
+    j.r = r + b.off;
+    j.off = b.off;
+    j.nrows = b.n;
+    j.slot0 = b.slot_main;
+    j.block = b.off < h.split ? 0 : 1;
+    j.blocks = job_blocks(b.n);
+    blocks += j.blocks;
+    if (b.edge_free) {
+      j.ev = b.ev.p;
+      j.eh = X::eh(b);
+      continue;
+    }
+    j.rp = b.o_main.m.row_ptr.p;
+    j.col = b.o_main.m.col.p;
+    j.val = X::v(b.o_main);
+    j.C = b.o_main.C;
+    j.grad = b.j == 1;
     if (b.j == 2) {
-      const XCsr& ul = b.o_ul;
-      q(k_hx_out<TP, TP, TP>, grid_for(ul.m.nrows), TPB, ul.m.row_ptr.p, ul.m.col.p, X::v(ul), ul.C, 0, xs,
-        (const TP*)slots, X::dinv(l0), nx, b.slot_tl, X::sl(b), (const TP*)X::t(b), X::u(b), ul.m.nrows, 0, S);
-      const XCsr& od = b.o_d;
-      q(k_hx_out<TP, TP, TIN>, grid_for(od.m.nrows), TPB, od.m.row_ptr.p, od.m.col.p, X::v(od), od.C, 0,
-        (const TP*)X::u(b), (const TP*)nullptr, (const TP*)nullptr, nx, 0, sb, rb, zb, od.m.nrows, 0, S);
-      q(k_hx_out<TP, TP, TIN>, grid_for(om.m.nrows), TPB, om.m.row_ptr.p, om.m.col.p, X::v(om), om.C, 0, xs,
-        (const TP*)slots, X::dinv(l0), nx, b.slot_main, (const TP*)nullptr, (const TIN*)nullptr, zb,
-        om.m.nrows, 1, S);
-    } else if (b.edge_free) {
-      q(k_hx_out_edge<TP, TIN, D>, grid_for(b.n), TPB, (const int32_t*)b.ev.p, X::eh(b), xs, (const TP*)slots,
-        X::dinv(l0), nx, b.slot_main, sb, rb, zb, b.n, S);
-    } else {
-      q(k_hx_out<TP, TP, TIN>, grid_for(om.m.nrows), TPB, om.m.row_ptr.p, om.m.col.p, X::v(om), om.C,
-        b.j == 1 ? 1 : 0, xs, (const TP*)slots, X::dinv(l0), nx, b.slot_main, sb, rb, zb, om.m.nrows, 0, S);
+      j.drp = b.o_d.m.row_ptr.p;
+      j.dcol = b.o_d.m.col.p;
+      j.dval = X::v(b.o_d);
+      j.sl = X::sl(b);
+      j.t = X::t(b);
     }
   }
+  const ChebVecs<TP> c{X::zt(h), X::res(h), X::d(h), X::zc(h), h.coef.p, k};
+  q(k_hx_out<TP, TIN, D, MODE>, blocks, TPB, out, xs, (const TP*)slots, X::dinv(l0), nx, c, S);
 }
 
 // y = P x: FP64 values on the FP64 path, the symmetric FP32 copy otherwise.
@@ -2786,23 +2905,18 @@ void pc_spmv(Enq& q, Hx& h, const TP* x, TP* y, const MinresS* S) {
 template <class TIN, class TP, class TOUT, int D>
 void hx_apply_d(Enq& q, Hx& h, const TIN* r, TOUT* z, const MinresS* S, double* part) {
   using X = Sel<TP>;
-  hx_core_d<TIN, TP, D>(q, h, r, S);
   if (h.cheb_m <= 1) {
+    hx_core_d<TIN, TP, D>(q, h, r, S);
     q(k_hx_final<TIN, TP, TOUT>, red_grid(h.N), TPB, r, (const TP*)X::zt(h), z, h.n, h.N, S, part);
     return;
   }
-  TP* res = X::res(h);
-  TP* d = X::d(h);
-  TP* zc = X::zc(h);
-  TP* w = X::w(h);
-  const double* coef = h.coef.p;
-  q(k_hxc_first<TP>, grid_for(h.n), TPB, (const TP*)X::zt(h), res, d, zc, h.n, h.split, coef, S);
+  hx_core_d<TIN, TP, D, 1>(q, h, r, S);
   for (int k = 0; k + 1 < h.cheb_m; ++k) {
-    pc_spmv<TP>(q, h, (const TP*)d, w, S);
-    hx_core_d<TP, TP, D>(q, h, (const TP*)w, S);
-    q(k_hxc_step<TP>, grid_for(h.n), TPB, (const TP*)X::zt(h), res, d, zc, h.n, h.split, coef, k, S);
+    pc_spmv<TP>(q, h, (const TP*)X::d(h), X::w(h), S);
+    hx_core_d<TP, TP, D, 2>(q, h, (const TP*)X::w(h), S, k);
   }
-  q(k_hxc_final<TIN, TP, TOUT>, red_grid(h.N), TPB, r, (const TP*)zc, (const TP*)d, z, h.n, h.N, S, part);
+  q(k_hxc_final<TIN, TP, TOUT>, red_grid(h.N), TPB, r, (const TP*)X::zc(h), (const TP*)X::d(h), z, h.n, h.N, S,
+    part);
 }
 
 template <class TIN, class TP, class TOUT>
