@@ -132,6 +132,12 @@ __device__ __host__ __forceinline__ int stencil_point(const int* diff) {
 // ---------------------------------------------------------------------------
 // the V-cycle on stencil levels: one thread per (vertex, slot)
 // ---------------------------------------------------------------------------
+// blockIdx.y is the slot and gridDim.x a multiple of the 8 XCDs (slot_grid), so
+// that an XCD works on the same contiguous range of vertices for every slot and
+// its L2 fetches the operator once. (A thread that took all 5 slots of its
+// vertex read the operator once by itself and was slower, 16.4 us a sweep at
+// 65^3: its slots' loads follow each other.)
+
 // x = dinv r (the first sweep from x = 0)
 template <class TP>
 __global__ void __launch_bounds__(TPB) k_st_scale(const TP* __restrict__ dinv, const TP* __restrict__ r,
@@ -143,10 +149,10 @@ __global__ void __launch_bounds__(TPB) k_st_scale(const TP* __restrict__ dinv, c
   x[t] = dinv[t % nb] * r[t];
 }
 
-// The sweep family, one thread per (vertex, slot). The operator is
-// symmetric, so a row's -delta entries are read from the +delta diagonals at
-// the neighbour (A(i, i - o) = A(i - o, i)): only the diagonal and the 2^d - 1
-// +delta diagonals are fetched. MODE selects the iterate the sweep starts from:
+// The sweep family. The operator is symmetric, so a row's -delta entries are
+// read from the +delta diagonals at the neighbour (A(i, i - o) = A(i - o, i)):
+// only the diagonal and the 2^d - 1 +delta diagonals are fetched. MODE selects
+// the iterate the sweep starts from:
 //   0: out = x + dinv (r - A x)                  (a weighted Jacobi sweep)
 //   1: out = r - A x, 0 on dead rows             (the residual)
 //   2: the sweep from x = dinv r                 (the first two pre-sweeps in one)
@@ -161,16 +167,15 @@ __device__ __forceinline__ TP st_iterate(int j, const TP* __restrict__ x, const 
 template <class TP, int D, int MODE, bool FINE>
 __global__ void __launch_bounds__(TPB) k_st_sweep(const TP* __restrict__ A, const TP* __restrict__ dinv,
                                                   const TP* __restrict__ r, const TP* __restrict__ x,
-                                                  TP* __restrict__ out, Box b, unsigned nv, const MinresS* S) {
+                                                  TP* __restrict__ out, Box b, const MinresS* S) {
   constexpr int H = (1 << D) - 1;
   if (skip(S)) return;
-  const unsigned t = xcd_block() * blockDim.x + threadIdx.x;
+  const unsigned i = xcd_block() * blockDim.x + threadIdx.x;
   const unsigned nb = (unsigned)b.nb;
-  if (t >= nb * nv) return;
-  const unsigned base = t / nb * nb;  // the slot's vectors
-  const unsigned i = t - base;
+  if (i >= nb) return;
+  const size_t base = (size_t)blockIdx.y * nb;  // the slot's vectors
   r += base;
-  x += base;
+  if (MODE != 2) x += base;
   const TP xi = st_iterate<TP, MODE>((int)i, x, dinv, r);
   TP acc = A[i] * xi;
 #pragma unroll
@@ -188,7 +193,7 @@ __global__ void __launch_bounds__(TPB) k_st_sweep(const TP* __restrict__ A, cons
   }
   const TP d = dinv[i];
   const TP res = r[i] - acc;
-  out[t] = MODE == 1 ? (d != TP(0) ? res : TP(0)) : xi + d * res;
+  (out + base)[i] = MODE == 1 ? (d != TP(0) ? res : TP(0)) : xi + d * res;
 }
 
 // rc = P^T ef on the live coarse vertices (0 elsewhere): coarse vertex w
@@ -196,17 +201,12 @@ __global__ void __launch_bounds__(TPB) k_st_sweep(const TP* __restrict__ A, cons
 template <class TP, int D>
 __global__ void __launch_bounds__(TPB) k_st_restrict(const TP* __restrict__ ef, TP* __restrict__ rc,
                                                      const uint8_t* __restrict__ live_c, Box fb, Box cb,
-                                                     unsigned nv, const MinresS* S) {
+                                                     const MinresS* S) {
   constexpr int H = (1 << D) - 1;
   if (skip(S)) return;
-  const unsigned t = xcd_block() * blockDim.x + threadIdx.x;
-  if (t >= (unsigned)cb.nb * nv) return;
-  const unsigned v = t / (unsigned)cb.nb;
-  const unsigned w = t - v * (unsigned)cb.nb;
-  if (!live_c[w]) {
-    rc[t] = TP(0);
-    return;
-  }
+  const unsigned w = xcd_block() * blockDim.x + threadIdx.x;
+  if (w >= (unsigned)cb.nb) return;
+  const TP* __restrict__ e = ef + (size_t)blockIdx.y * (unsigned)fb.nb;
   int wc[D];
   {
     unsigned r = w;
@@ -216,12 +216,13 @@ __global__ void __launch_bounds__(TPB) k_st_restrict(const TP* __restrict__ ef, 
       r /= (unsigned)(cb.g + 1);
     }
   }
+  const bool live = live_c[w];
   TP acc = TP(0);
 #pragma unroll
   for (int s = 0; s <= 2 * H; ++s) {
     const int mask = s <= H ? s : s - H;
     const int sg = s <= H ? 1 : -1;
-    bool in = true;
+    bool in = live;
     int k = 0;
 #pragma unroll
     for (int a = 0; a < D; ++a) {
@@ -229,35 +230,30 @@ __global__ void __launch_bounds__(TPB) k_st_restrict(const TP* __restrict__ ef, 
       in = in && c >= 0 && c <= fb.g;
       k += c * fb.st[a];
     }
-    if (in) acc += (s == 0 ? TP(1) : TP(0.5)) * ef[v * (unsigned)fb.nb + (unsigned)k];
+    acc += (in ? (s == 0 ? TP(1) : TP(0.5)) : TP(0)) * e[in ? (unsigned)k : 0u];
   }
-  rc[t] = acc;
+  (rc + (size_t)blockIdx.y * (unsigned)cb.nb)[w] = acc;
 }
 
 // xf += P xc on the live fine vertices (dinv_f != 0).
 template <class TP, int D>
 __global__ void __launch_bounds__(TPB) k_st_prolong(const TP* __restrict__ xc, TP* __restrict__ xf,
                                                     const TP* __restrict__ dinv_f, Box fb, Box cb,
-                                                    unsigned nv, const MinresS* S) {
+                                                    const MinresS* S) {
   if (skip(S)) return;
-  const unsigned t = xcd_block() * blockDim.x + threadIdx.x;
-  if (t >= (unsigned)fb.nb * nv) return;
-  const unsigned v = t / (unsigned)fb.nb;
-  const unsigned k = t - v * (unsigned)fb.nb;
+  const unsigned k = xcd_block() * blockDim.x + threadIdx.x;
+  if (k >= (unsigned)fb.nb) return;
   if (dinv_f[k] == TP(0)) return;
-  xc += v * (unsigned)cb.nb;
-  unsigned r = k;
-  int lo = 0, hi = 0;
-  bool odd = false;
+  unsigned r = k, lo = 0, hi = 0;
 #pragma unroll
   for (int a = 0; a < D; ++a) {
-    const int c = (int)(r % (unsigned)(fb.g + 1));
+    const unsigned c = r % (unsigned)(fb.g + 1);
     r /= (unsigned)(fb.g + 1);
-    lo += (c >> 1) * cb.st[a];
-    hi += ((c >> 1) + (c & 1)) * cb.st[a];
-    odd = odd || (c & 1);
+    lo += (c >> 1) * (unsigned)cb.st[a];
+    hi += ((c + 1) >> 1) * (unsigned)cb.st[a];
   }
-  xf[t] += odd ? TP(0.5) * (xc[lo] + xc[hi]) : xc[lo];
+  xc += (size_t)blockIdx.y * (unsigned)cb.nb;
+  (xf + (size_t)blockIdx.y * (unsigned)fb.nb)[k] += TP(0.5) * (xc[lo] + xc[hi]);
 }
 
 // x = C r on the coarsest box, C dense (nb x nb, row-major, zero on dead
@@ -2752,14 +2748,17 @@ struct LevelTiles {
   bool use(const Hx& h) const { return d <= 3 && h.sweeps == 2 && std::max(down, up) * h.nv <= (d == 3 ? 512 : 2048); }
 };
 
+// The grid of the plain level kernels: vertices by slots.
+inline dim3 slot_grid(int64_t vertices, unsigned nv) { return dim3((grid_for(vertices) + 7) / 8 * 8, nv); }
+
 template <class TP, int D, bool FINE>
 void sweep_launch(Enq& q, int mode, const MgLevel& l, const TP* A, const TP* dinv, const TP* r, const TP* x,
                   TP* out, unsigned nv, const MinresS* S) {
-  const unsigned g = grid_for((int64_t)l.box.nb * nv);
+  const dim3 g = slot_grid(l.box.nb, nv);
   switch (mode) {
-    case 0: q(k_st_sweep<TP, D, 0, FINE>, g, TPB, A, dinv, r, x, out, l.box, nv, S); break;
-    case 1: q(k_st_sweep<TP, D, 1, FINE>, g, TPB, A, dinv, r, x, out, l.box, nv, S); break;
-    default: q(k_st_sweep<TP, D, 2, FINE>, g, TPB, A, dinv, r, x, out, l.box, nv, S); break;
+    case 0: q(k_st_sweep<TP, D, 0, FINE>, g, TPB, A, dinv, r, x, out, l.box, S); break;
+    case 1: q(k_st_sweep<TP, D, 1, FINE>, g, TPB, A, dinv, r, x, out, l.box, S); break;
+    default: q(k_st_sweep<TP, D, 2, FINE>, g, TPB, A, dinv, r, x, out, l.box, S); break;
   }
 }
 
@@ -2815,10 +2814,10 @@ TP* vcycle(Enq& q, Hx& h, size_t i, const MinresS* S) {
     }
   }
   sweep(1, X::e(l));
-  q(k_st_restrict<TP, D>, grid_for((int64_t)c.box.nb * nv), TPB, (const TP*)X::e(l), X::r(c),
-    (const uint8_t*)c.alive.p, l.box, c.box, nv, S);
+  q(k_st_restrict<TP, D>, slot_grid(c.box.nb, nv), TPB, (const TP*)X::e(l), X::r(c), (const uint8_t*)c.alive.p,
+    l.box, c.box, S);
   TP* xc = vcycle<TP, D>(q, h, i + 1, S);
-  q(k_st_prolong<TP, D>, grid_for(nbv), TPB, (const TP*)xc, x, dinv, l.box, c.box, nv, S);
+  q(k_st_prolong<TP, D>, slot_grid(l.box.nb, nv), TPB, (const TP*)xc, x, dinv, l.box, c.box, S);
   for (int s = 0; s < h.sweeps; ++s) {
     sweep(0, y);
     std::swap(x, y);
