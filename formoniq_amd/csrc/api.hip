@@ -646,9 +646,11 @@ void problem_assemble_from_elements(Problem& P) {
   }
   if (P.sys.P.nnz) coo_plan_values(ctx, P.pc_plan, P.el.p, P.sys.P.val.p, nullptr);
   problem_multigrid(P);
-  // the FP32/FP16 copies are made for mixed and FP64_PC32 problems, the FP64
-  // SELL copy for FP64 ones; either is refreshed once made
-  if (P.opts.precision != FEEC_PREC_FP64 || P.sys.val32.p) kkt_refresh_fp32(P.sys);
+  // the FP32/FP16 copies are made for mixed and FP64_PC32 problems (the latter
+  // need none with the multigrid blocks), the FP64 SELL copy for FP64 ones;
+  // either is refreshed once made
+  if (P.opts.precision == FEEC_PREC_MIXED || (P.opts.precision == FEEC_PREC_FP64_PC32 && !P.hx) || P.sys.val32.p)
+    kkt_refresh_fp32(P.sys);
   if (!P.hx) {
     if ((P.opts.precision == FEEC_PREC_FP64 && P.opts.precond_storage == FEEC_PC_STORE_SELL) ||
         P.sys.Psell64.p)

@@ -1931,11 +1931,11 @@ static void bind_fp32(KktSystem& s, MinresWork<float>& w, int storage) {
 // solve's preconditioner without its restarts). Without a polynomial, or
 // without the SELL copy, the FP64 binding on P's CSR values.
 static void bind_pc32(KktSystem& s, MinresWork<double>& w) {
-  if (!s.val32.p) kkt_refresh_fp32(s);
   if (s.hx) {
     bind_hx(s, w, true);
     return;
   }
+  if (!s.val32.p) kkt_refresh_fp32(s);
   w.hx = nullptr;
   const int m = (s.P.nnz > 0 && s.cheb_m > 0 && s.cheb.p) ? s.cheb_m : 0;
   if (m == 0 || !(s.Psell.p || s.Psell_v16.p) || !s.sdinv32.p) {

@@ -1289,6 +1289,176 @@ __global__ void k_sym_single(const double* __restrict__ val, const int32_t* __re
   if (q < n) out[q] = (float)(0.5 * (val[q] + val[tpos[q]]));
 }
 
+// --- P in slices with shared offset lists --------------------------------------
+// On a grid numbered by rows, P's rows repeat lists of column offsets: inside, a
+// row's list depends on its simplex's direction alone, and only next to the
+// first planes, where the counts per vertex change, is each list its own (3% of
+// the rows at 64^3). So a row keeps the number of its list in place of its
+// columns: 4 B an entry in FP32 against 6, 8 in FP64 against 12. Rows are sorted
+// by length in windows of 256 and stored 64 to a slice, entry j of the slice's
+// rows side by side, one lane a row; rows and vectors keep their numbers.
+constexpr int SELL_WIN = 256;
+constexpr int kMaxLists = 1 << 17;     // lists a matrix may have (and at most n / 8)
+constexpr int kListSlots = 2 * kMaxLists;  // of the hash table they are found by
+
+__device__ __forceinline__ unsigned long long mix64(unsigned long long h, unsigned long long v) {
+  h ^= v + 0x9E3779B97F4A7C15ull + (h << 6) + (h >> 2);
+  h *= 0xBF58476D1CE4E5B9ull;
+  return h ^ (h >> 29);
+}
+// slot[row]: the place of the row's list in the table; *bad: the table is full.
+// keys: 0 free; rep: the smallest row of the list.
+__global__ void k_list_find(const int64_t* rp, const int32_t* col, int64_t n, unsigned long long* keys,
+                            unsigned int* rep, int32_t* slot, int32_t* len, int* bad) {
+  const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (r >= n) return;
+  const int64_t b = rp[r], e = rp[r + 1];
+  unsigned long long h = mix64(0x2545F4914F6CDD1Dull, (unsigned long long)(e - b));
+  for (int64_t p = b; p < e; ++p) h = mix64(h, (unsigned long long)(col[p] - r));
+  if (h == 0) h = 1;
+  len[r] = (int32_t)(e - b);
+  slot[r] = 0;
+  for (int probe = 0; probe < 64; ++probe) {
+    const int s = (int)((h + probe) % kListSlots);
+    unsigned long long have = __atomic_load_n(&keys[s], __ATOMIC_RELAXED);
+    if (have == 0) have = atomicCAS(&keys[s], 0ull, h);
+    if (have == 0 || have == h) {
+      if (__atomic_load_n(&rep[s], __ATOMIC_RELAXED) > (unsigned)r) atomicMin(&rep[s], (unsigned)r);
+      slot[r] = s;
+      return;
+    }
+  }
+  atomicOr(bad, 1);
+}
+// ids of the occupied slots, in slot order; count[0] lists, count[1] the longest row
+__global__ void __launch_bounds__(TPB) k_list_ids(const unsigned long long* keys, const unsigned int* rep,
+                                                  const int32_t* len, int32_t* id, int* count) {
+  __shared__ int base[TPB];
+  __shared__ int longest;
+  constexpr int PER = kListSlots / TPB;
+  const int t = threadIdx.x;
+  if (t == 0) longest = 0;
+  int c = 0, top = 0;
+  for (int i = 0; i < PER; ++i)
+    if (keys[t * PER + i]) {
+      ++c;
+      top = max(top, len[rep[t * PER + i]]);
+    }
+  base[t] = c;
+  __syncthreads();
+  atomicMax(&longest, top);
+  if (t == 0) {
+    int s = 0;
+    for (int i = 0; i < TPB; ++i) {
+      const int x = base[i];
+      base[i] = s;
+      s += x;
+    }
+    count[0] = s;
+  }
+  __syncthreads();
+  int at = base[t];
+  for (int i = 0; i < PER; ++i) id[t * PER + i] = keys[t * PER + i] ? at++ : -1;
+  if (t == 0) count[1] = longest;
+}
+// tab[id * width + j]: the list's offsets, from its smallest row
+__global__ void k_list_table(const int64_t* rp, const int32_t* col, const unsigned long long* keys,
+                             const unsigned int* rep, const int32_t* id, int width, int32_t* tab) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= kListSlots || !keys[s]) return;
+  const int64_t r = rep[s], b = rp[r];
+  const int m = (int)(rp[r + 1] - b);
+  for (int j = 0; j < width; ++j) tab[(int64_t)id[s] * width + j] = j < m ? (int32_t)(col[b + j] - r) : 0;
+}
+// One block per window: its rows by length, longest first (rows of one length in
+// their order), their lists, and the width of each of its slices; bad: a row
+// that differs from its list (two lists of one hash).
+__global__ void __launch_bounds__(SELL_WIN) k_list_sort(const int64_t* rp, const int32_t* col, const int32_t* len,
+                                                        const int32_t* slot, const int32_t* id, const int32_t* tab,
+                                                        int width, int64_t n, int32_t* perm, int32_t* list,
+                                                        unsigned long long* entries, int64_t slices, int* bad) {
+  __shared__ int sl[SELL_WIN];
+  __shared__ int top[SELL_WIN / 64];
+  const int t = threadIdx.x;
+  const int64_t r = blockIdx.x * (int64_t)SELL_WIN + t;
+  const int m = r < n ? len[r] : -1;
+  sl[t] = m;
+  if (t < SELL_WIN / 64) top[t] = 0;
+  __syncthreads();
+  int at = 0;
+  for (int i = 0; i < SELL_WIN; ++i) at += sl[i] > m || (sl[i] == m && i < t);
+  const int l = r < n ? id[slot[r]] : 0;
+  perm[blockIdx.x * (int64_t)SELL_WIN + at] = r < n ? (int32_t)r : -1;
+  list[blockIdx.x * (int64_t)SELL_WIN + at] = l;
+  if (m > 0) atomicMax(&top[at / 64], m);
+  if (r < n) {
+    bool same = true;
+    for (int j = 0; j < m; ++j) same = same && tab[(int64_t)l * width + j] == (int32_t)(col[rp[r] + j] - r);
+    if (!same) atomicOr(bad, 1);
+  }
+  __syncthreads();
+  if (t < SELL_WIN / 64) {
+    const int64_t s = blockIdx.x * (int64_t)(SELL_WIN / 64) + t;
+    if (s < slices) entries[s] = 64ull * (unsigned long long)top[t];
+    if (s == slices - 1) entries[slices] = 0;  // the scan ends on the total
+  }
+}
+// place[p]: where CSR entry p lies in the slices
+__global__ void k_list_places(const int64_t* rp, const int32_t* perm, const int64_t* ptr, int64_t npad,
+                              int32_t* place) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= npad) return;
+  const int32_t r = perm[i];
+  if (r < 0) return;
+  const int64_t b = rp[r], base = ptr[i >> 6] + (i & 63);
+  for (int64_t p = b; p < rp[r + 1]; ++p) place[p] = (int32_t)(base + 64 * (p - b));
+}
+// the slices' values: P's own (FP64), or (P + P^T) / 2 rounded once (FP32)
+__global__ void k_list_values(const double* val, const int32_t* place, int64_t nnz, double* out) {
+  const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (p < nnz) out[place[p]] = val[p];
+}
+__global__ void k_list_values(const double* val, const int32_t* tpos, const int32_t* place, int64_t nnz,
+                              float* out) {
+  const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (p < nnz) out[place[p]] = (float)(0.5 * (val[p] + val[tpos[p]]));
+}
+// y = P x on the slices, one lane a row, its entries four at a time in their order
+template <class TP>
+__global__ void __launch_bounds__(TPB) k_pc_lists(const int64_t* __restrict__ ptr, const int32_t* __restrict__ perm,
+                                                  const int32_t* __restrict__ list, const int32_t* __restrict__ tab,
+                                                  int width, const TP* __restrict__ val, const TP* __restrict__ x,
+                                                  TP* __restrict__ y, int64_t npad, const MinresS* S) {
+  if (skip(S)) return;
+  const int64_t i = xcd_block() * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= npad) return;
+  const int32_t row = perm[i];
+  if (row < 0) return;  // past the last row: no list is its own
+  const int64_t base = ptr[i >> 6];
+  const int w = (int)((ptr[(i >> 6) + 1] - base) >> 6);
+  const TP* __restrict__ v = val + base + (i & 63);
+  const int4* __restrict__ t = reinterpret_cast<const int4*>(tab + (int64_t)list[i] * width);
+  const TP* __restrict__ xr = x + row;
+  TP acc = TP(0);
+  int j = 0;
+  for (; j + 4 <= w; j += 4) {
+    const int4 o = t[j / 4];
+    const TP a = v[64 * j], b = v[64 * (j + 1)], c = v[64 * (j + 2)], d = v[64 * (j + 3)];
+    const TP xa = xr[o.x], xb = xr[o.y], xc = xr[o.z], xd = xr[o.w];
+    acc += a * xa;
+    acc += b * xb;
+    acc += c * xc;
+    acc += d * xd;
+  }
+  if (j < w) {
+    const int4 o = t[j / 4];
+    acc += v[64 * j] * xr[o.x];
+    if (j + 1 < w) acc += v[64 * (j + 1)] * xr[o.y];
+    if (j + 2 < w) acc += v[64 * (j + 2)] * xr[o.z];
+  }
+  y[row] = acc;
+}
+
 // y = P32 x, columns as int16 offsets from the row or int32; LPR lanes per row.
 // Each lane takes its entries U at a time (loads, then gathers, then the
 // products added in entry order): more loads in flight per lane and the same
@@ -1650,6 +1820,17 @@ struct Hx {
   DBuf<float> P32;              // exactly symmetric FP32 copy: the FP32 Chebyshev steps' P
   DBuf<int32_t> P_tpos;         // entry of P's transpose, per entry
   DBuf<int16_t> P_col16;        // column offsets from the row, when all fit 16 bits
+  bool P_narrow = false;        // they do
+  // P in slices with shared offset lists (k_pc_lists), in the problem's precision
+  struct Lists {
+    bool on = false;
+    int width = 0;
+    int64_t npad = 0, entries = 0;
+    DBuf<int64_t> ptr;
+    DBuf<int32_t> perm, list, tab, place;
+    DBuf<float> v32;
+    DBuf<double> v64;
+  } lists;
   DBuf<double> coef, pvec, part, lz;
   DBuf<double> res64, d64, zc64, w64;
   DBuf<float> res32, d32, zc32, w32;
@@ -2240,9 +2421,69 @@ void bind_pc_matrix(Hx& h, const KktSystem& s) {
   h.P_col = s.P.col.p;
   h.P_val = s.P.val.p;
   h.P_nnz = s.P.nnz;
-  if (h.cheb_m > 1 && h.P_tpos.p && s.P.nnz)
-    k_sym_single<<<grid_for(s.P.nnz), TPB, 0, h.ctx->stream>>>(s.P.val.p, h.P_tpos.p, s.P.nnz, h.P32.p);
+  if (h.cheb_m > 1 && s.P.nnz) {
+    hipStream_t st = h.ctx->stream;
+    const unsigned g = grid_for(s.P.nnz);
+    if (h.lists.v32.p)
+      k_list_values<<<g, TPB, 0, st>>>(s.P.val.p, h.P_tpos.p, h.lists.place.p, s.P.nnz, h.lists.v32.p);
+    if (h.lists.v64.p) k_list_values<<<g, TPB, 0, st>>>(s.P.val.p, h.lists.place.p, s.P.nnz, h.lists.v64.p);
+    if (h.P32.p) k_sym_single<<<g, TPB, 0, st>>>(s.P.val.p, h.P_tpos.p, s.P.nnz, h.P32.p);
+  }
   FEEC_HIP(hipGetLastError());
+}
+
+// P's slices (k_pc_lists), where its rows repeat few enough offset lists and
+// there are enough of them that one lane a row fills the chip.
+constexpr int64_t kListRows = 100000;
+void build_lists(Hx& h, const KktSystem& s) {
+  Ctx* ctx = h.ctx;
+  hipStream_t st = ctx->stream;
+  Hx::Lists& l = h.lists;
+  const int64_t n = s.P.nrows, nnz = s.P.nnz;
+  if (n < kListRows || n >= ((int64_t)1 << 31) - SELL_WIN) return;
+  DBuf<unsigned long long> keys(ctx, kListSlots);
+  DBuf<unsigned int> rep(ctx, kListSlots);
+  DBuf<int32_t> id(ctx, kListSlots), slot(ctx, n), len(ctx, n);
+  DBuf<int> count(ctx, 4);  // lists, longest row, bad
+  FEEC_HIP(hipMemsetAsync(keys.p, 0, kListSlots * sizeof(unsigned long long), st));
+  FEEC_HIP(hipMemsetAsync(rep.p, 0xff, kListSlots * sizeof(unsigned int), st));
+  k_zero_i32<<<1, 64, 0, st>>>(count.p, 4);
+  k_list_find<<<grid_for(n), TPB, 0, st>>>(s.P.row_ptr.p, s.P.col.p, n, keys.p, rep.p, slot.p, len.p, count.p + 2);
+  k_list_ids<<<1, TPB, 0, st>>>(keys.p, rep.p, len.p, id.p, count.p);
+  FEEC_HIP(hipGetLastError());
+  int hc[4] = {0, 0, 0, 0};
+  copy_to_host(ctx, hc, count.p, sizeof(hc));
+  if (hc[2] || hc[0] > kMaxLists || hc[0] > n / 8 || hc[1] > 1024) return;
+  l.width = (hc[1] + 3) / 4 * 4;
+  l.tab.alloc(ctx, std::max<int64_t>((int64_t)hc[0] * l.width, 4));
+  k_list_table<<<grid_for(kListSlots), TPB, 0, st>>>(s.P.row_ptr.p, s.P.col.p, keys.p, rep.p, id.p, l.width,
+                                                     l.tab.p);
+  const int64_t windows = (n + SELL_WIN - 1) / SELL_WIN, slices = windows * (SELL_WIN / 64);
+  l.npad = windows * SELL_WIN;
+  l.perm.alloc(ctx, l.npad);
+  l.list.alloc(ctx, l.npad);
+  l.ptr.alloc(ctx, slices + 1);
+  DBuf<unsigned long long> entries(ctx, slices + 1);
+  k_list_sort<<<(unsigned)windows, SELL_WIN, 0, st>>>(s.P.row_ptr.p, s.P.col.p, len.p, slot.p, id.p, l.tab.p,
+                                                      l.width, n, l.perm.p, l.list.p, entries.p, slices,
+                                                      count.p + 2);
+  FEEC_HIP(hipGetLastError());
+  exclusive_scan_counts(ctx, entries.p, l.ptr.p, slices + 1);
+  copy_to_host(ctx, &l.entries, l.ptr.p + slices, sizeof(int64_t));
+  copy_to_host(ctx, hc, count.p, sizeof(hc));
+  if (hc[2] || l.entries >= ((int64_t)1 << 31)) return;
+  l.place.alloc(ctx, nnz);
+  k_list_places<<<grid_for(l.npad), TPB, 0, st>>>(s.P.row_ptr.p, l.perm.p, l.ptr.p, l.npad, l.place.p);
+  FEEC_HIP(hipGetLastError());
+  // the padding's zeros stay: a refresh writes the entries' places alone
+  if (h.spectrum_fp32) {
+    l.v32.alloc(ctx, std::max<int64_t>(l.entries, 1));
+    FEEC_HIP(hipMemsetAsync(l.v32.p, 0, l.v32.n * sizeof(float), st));
+  } else {
+    l.v64.alloc(ctx, std::max<int64_t>(l.entries, 1));
+    FEEC_HIP(hipMemsetAsync(l.v64.p, 0, l.v64.n * sizeof(double), st));
+  }
+  l.on = true;
 }
 
 // The pattern side of P's FP32 copy: the transpose entry of every entry (P is
@@ -2253,9 +2494,13 @@ void build_pc_single(Hx& h, const KktSystem& s) {
   Ctx* ctx = h.ctx;
   const int64_t n = s.P.nrows, nnz = s.P.nnz;
   h.P_tpos.alloc(ctx, std::max<int64_t>(nnz, 1));
-  h.P32.alloc(ctx, std::max<int64_t>(nnz, 1));
+  h.P32.reset();
   h.P_col16.reset();
-  if (!nnz) return;
+  h.P_narrow = true;
+  if (!nnz) {
+    h.P32.alloc(ctx, 1);
+    return;
+  }
   DBuf<int16_t> c16(ctx, nnz);
   // flags[0]: some entry has no transpose; flags[1]: some offset is beyond 16 bits
   DBuf<int> flags(ctx, 2);
@@ -2266,7 +2511,13 @@ void build_pc_single(Hx& h, const KktSystem& s) {
   int hf[2] = {0, 0};
   copy_to_host(ctx, hf, flags.p, sizeof(hf));
   FEEC_REQUIRE(hf[0] == 0, FEEC_E_DEVICE, "preconditioner matrix is not structurally symmetric");
-  if (hf[1] == 0) h.P_col16 = std::move(c16);
+  h.P_narrow = hf[1] == 0;
+  build_lists(h, s);
+  // the CSR copy: where there are no slices, and for an FP64 problem's FP32 applications
+  if (!h.lists.v32.p) {
+    h.P32.alloc(ctx, nnz);
+    if (h.P_narrow) h.P_col16 = std::move(c16);
+  }
 }
 }  // namespace
 
@@ -2566,7 +2817,7 @@ Hx* hx_create(Geom& g, int bc, int k, const KktSystem& s, int sweeps, int cheb_m
       if (x->m.nnz) bytes += x->m.nnz * 4 * (1 + x->C) + x->m.nrows * 8;
   launches += 2;
   if (h->cheb_m > 1) {
-    bytes = bytes * h->cheb_m + (h->cheb_m - 1) * (s.P.nnz * (h->P_col16.p ? 6 : 8) + h->n * 28) + h->n * 12;
+    bytes = bytes * h->cheb_m + (h->cheb_m - 1) * ((h->lists.on ? 4 * h->lists.entries : s.P.nnz * (h->P_narrow ? 6 : 8)) + h->n * 28) + h->n * 12;
     launches = launches * h->cheb_m + (h->cheb_m - 1) + 1;
   }
   h->bytes32 = bytes;
@@ -2888,6 +3139,17 @@ void hx_core_d(Enq& q, Hx& h, const TIN* r, const MinresS* S, int k = 0) {
 template <class TP>
 void pc_spmv(Enq& q, Hx& h, const TP* x, TP* y, const MinresS* S) {
   const unsigned g = grid_for(h.n * 4);
+  const Hx::Lists& l = h.lists;
+  const TP* lv = nullptr;
+  if constexpr (std::is_same_v<TP, double>)
+    lv = l.v64.p;
+  else
+    lv = l.v32.p;
+  if (l.on && lv) {
+    q(k_pc_lists<TP>, (grid_for(l.npad) + 7) / 8 * 8, TPB, (const int64_t*)l.ptr.p, (const int32_t*)l.perm.p,
+      (const int32_t*)l.list.p, (const int32_t*)l.tab.p, l.width, lv, x, y, l.npad, S);
+    return;
+  }
   if constexpr (std::is_same_v<TP, double>) {
     q(k_pc_spmv<double, double, 4, 2>, g, TPB, h.P_rp, h.P_col, h.P_val, x, y, h.n, S);
   } else {
@@ -3181,7 +3443,7 @@ void hx_kernel_times(Hx& h, int reps, bool use_graph, double out[4]) {
 
 void hx_info(const Hx& h, int* cheb_m, double lam[2], int* column_bytes) {
   if (cheb_m) *cheb_m = h.cheb_m;
-  if (column_bytes) *column_bytes = h.P_col16.p ? 2 : 4;
+  if (column_bytes) *column_bytes = h.P_narrow ? 2 : 4;
   if (lam) {
     lam[0] = h.lam[0];
     lam[1] = h.lam[1];
