@@ -1022,7 +1022,11 @@ __device__ __forceinline__ int find_job(const J* jobs, int n, unsigned& blk) {
 }
 
 // y[v * ny + row] = sum_p val[p * C + v] x[col[p]] for v < C; lpr lanes (1 or 4)
-// share a row, entries strided over them, summed by shuffles.
+// share a row, entries strided over them, summed by shuffles. All blocks' gathers
+// are one launch: on small grids each was bound by its launch (3D 27^3 grade 2:
+// 9 of them and the Chebyshev step, 49.8 ms a solve and assembly; in one each way
+// 40.5), on large ones by the entries' values (64^3: 46 us alone with values read
+// one at a time, 29 with wide loads).
 template <class TX, class TP>
 struct GatherJob {
   const int64_t* rp;
@@ -1296,10 +1300,13 @@ __global__ void k_sym_single(const double* __restrict__ val, const int32_t* __re
 // the rows at 64^3). So a row keeps the number of its list in place of its
 // columns: 4 B an entry in FP32 against 6, 8 in FP64 against 12. Rows are sorted
 // by length in windows of 256 and stored 64 to a slice, entry j of the slice's
-// rows side by side, one lane a row; rows and vectors keep their numbers.
+// rows side by side, one lane a row; rows and vectors keep their numbers. Bound
+// by the matrix stream and the gathers of x: 64^3 in FP32 70.2 us as compressed
+// rows (206 MB), 59.9 so (144 MB); 33^3 in FP64 14.6 and 13.0.
 constexpr int SELL_WIN = 256;
 constexpr int kMaxLists = 1 << 17;     // lists a matrix may have (and at most n / 8)
 constexpr int kListSlots = 2 * kMaxLists;  // of the hash table they are found by
+static_assert(kListSlots % TPB == 0);
 
 __device__ __forceinline__ unsigned long long mix64(unsigned long long h, unsigned long long v) {
   h ^= v + 0x9E3779B97F4A7C15ull + (h << 6) + (h >> 2);
@@ -1330,36 +1337,31 @@ __global__ void k_list_find(const int64_t* rp, const int32_t* col, int64_t n, un
   }
   atomicOr(bad, 1);
 }
-// ids of the occupied slots, in slot order; count[0] lists, count[1] the longest row
+// ids of the occupied slots, a run per block; count[0] lists, count[1] the longest
+// row. (One block for the whole table took 1.9 ms: a lane's 1,024 reads in turn.)
 __global__ void __launch_bounds__(TPB) k_list_ids(const unsigned long long* keys, const unsigned int* rep,
                                                   const int32_t* len, int32_t* id, int* count) {
-  __shared__ int base[TPB];
-  __shared__ int longest;
-  constexpr int PER = kListSlots / TPB;
-  const int t = threadIdx.x;
+  __shared__ int wave[TPB / 64];
+  __shared__ int base, longest;
+  const int t = threadIdx.x, s = blockIdx.x * TPB + t;  // kListSlots is a multiple of TPB
   if (t == 0) longest = 0;
-  int c = 0, top = 0;
-  for (int i = 0; i < PER; ++i)
-    if (keys[t * PER + i]) {
-      ++c;
-      top = max(top, len[rep[t * PER + i]]);
-    }
-  base[t] = c;
+  const bool used = keys[s] != 0;
+  const unsigned long long votes = __ballot(used);
+  if (t % 64 == 0) wave[t / 64] = __popcll(votes);
   __syncthreads();
-  atomicMax(&longest, top);
+  if (used) atomicMax(&longest, len[rep[s]]);
   if (t == 0) {
-    int s = 0;
-    for (int i = 0; i < TPB; ++i) {
-      const int x = base[i];
-      base[i] = s;
-      s += x;
+    int all = 0;
+    for (int w = 0; w < TPB / 64; ++w) {
+      const int x = wave[w];
+      wave[w] = all;
+      all += x;
     }
-    count[0] = s;
+    base = all ? atomicAdd(&count[0], all) : 0;
   }
   __syncthreads();
-  int at = base[t];
-  for (int i = 0; i < PER; ++i) id[t * PER + i] = keys[t * PER + i] ? at++ : -1;
-  if (t == 0) count[1] = longest;
+  if (t == 0 && longest) atomicMax(&count[1], longest);
+  id[s] = used ? base + wave[t / 64] + __popcll(votes & ((1ull << (t % 64)) - 1)) : -1;
 }
 // tab[id * width + j]: the list's offsets, from its smallest row
 __global__ void k_list_table(const int64_t* rp, const int32_t* col, const unsigned long long* keys,
@@ -2433,8 +2435,12 @@ void bind_pc_matrix(Hx& h, const KktSystem& s) {
 }
 
 // P's slices (k_pc_lists), where its rows repeat few enough offset lists and
-// there are enough of them that one lane a row fills the chip.
-constexpr int64_t kListRows = 100000;
+// there are enough of them that one lane a row fills the chip. FP32, us a product
+// in slices / as compressed rows, 3D k = 1: 118 k rows 7.7 / 7.0, 185 k 9.8 / 10.5,
+// 301 k 13.4 / 14.3, 531 k 18.2 / 20.3; 3D k = 2: 146 k 12.0 / 9.5, 363 k 14.8 /
+// 14.4 with the application 410.7 / 413.9; 2D k = 1: 136 k 6.3 / 6.8, 642 k 11.0 /
+// 14.2. Building the slices adds 0.2-0.4 ms to a 3D set-up (64^3: 37.0 -> 37.4).
+constexpr int64_t kListRows = 150000;
 void build_lists(Hx& h, const KktSystem& s) {
   Ctx* ctx = h.ctx;
   hipStream_t st = ctx->stream;
@@ -2449,7 +2455,7 @@ void build_lists(Hx& h, const KktSystem& s) {
   FEEC_HIP(hipMemsetAsync(rep.p, 0xff, kListSlots * sizeof(unsigned int), st));
   k_zero_i32<<<1, 64, 0, st>>>(count.p, 4);
   k_list_find<<<grid_for(n), TPB, 0, st>>>(s.P.row_ptr.p, s.P.col.p, n, keys.p, rep.p, slot.p, len.p, count.p + 2);
-  k_list_ids<<<1, TPB, 0, st>>>(keys.p, rep.p, len.p, id.p, count.p);
+  k_list_ids<<<kListSlots / TPB, TPB, 0, st>>>(keys.p, rep.p, len.p, id.p, count.p);
   FEEC_HIP(hipGetLastError());
   int hc[4] = {0, 0, 0, 0};
   copy_to_host(ctx, hc, count.p, sizeof(hc));
@@ -2995,7 +3001,8 @@ struct LevelTiles {
   }
   // whether the level takes k_st_down / k_st_up: two sweeps, and no more
   // workgroups than run at once (two a CU in 3D; 2D's use fewer registers and
-  // recompute less)
+  // recompute less). On one side 21^3, 5 slots: 16 us against 26 in separate
+  // launches; on the other 65^3: 75 against 50.
   bool use(const Hx& h) const { return d <= 3 && h.sweeps == 2 && std::max(down, up) * h.nv <= (d == 3 ? 512 : 2048); }
 };
 
