@@ -642,18 +642,18 @@ def main():
         if tr.get("n_kkt") != n_kkt:
             tr = {}
     if mg is not None:
-        # int16 column offsets (or int32) and FP32 values per entry, 8-byte row
-        # pointers, x read and y written once per row
-        p_rows, p_nnz, cb = n_kkt, int(pc["nnz"]), int(pc["column_bytes"])
-        spmv_bytes = p_nnz * (cb + 4) + 8 * (p_rows + 1) + 8 * p_rows
+        # an FP32 value per entry; per row its number and its list's number, x read
+        # and y written once; the lists themselves (shared by the rows) not counted
+        p_rows, p_nnz = n_kkt, int(pc["nnz"])
+        spmv_bytes = p_nnz * 4 + 16 * p_rows + 8 * (p_rows // 64 + 1)
         achieved = spmv_bytes / mg["pc_spmv32"] / 1e9
         roof = {
-            "kernel": "k_pc_spmv32<short,4,2> (y = P x, the block-diagonal preconditioner matrix in FP32, "
-                      "4 lanes per row)",
+            "kernel": "k_pc_lists<float> (y = P x, the block-diagonal preconditioner matrix in FP32, "
+                      "64-row slices with shared column-offset lists, a lane per row)",
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": tr.get("pc_spmv32_hbm_bytes_per_launch"),
             "algorithmic_bytes_per_launch": spmv_bytes, "launch_seconds": mg["pc_spmv32"],
-            "rows": p_rows, "nnz": p_nnz, "column_bytes": cb,
+            "rows": p_rows, "nnz": p_nnz,
         }
         nb0 = (args.n + 1) ** 3
         nv = 5  # slots of one 3D k = 1 cycle: sigma's V, u's gradient V and its 3 vector copies
@@ -663,7 +663,7 @@ def main():
         achieved = sweep_bytes / mg["sweep_fine"] / 1e9
         sweep_roof = {
             "kernel": "k_st_sweep<float,3,0,true> (finest-level weighted-Jacobi sweep of the multigrid V-cycle "
-                      "on the Kuhn-stencil diagonals, 5 interleaved slots, FP32)",
+                      "on the Kuhn-stencil diagonals, 5 slots, FP32)",
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": tr.get("sweep_fine_hbm_bytes_per_launch"),
             "algorithmic_bytes_per_launch": sweep_bytes, "launch_seconds": mg["sweep_fine"],
