@@ -42,6 +42,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "cg_state.hpp"
 #include "feec_internal.hpp"
 #include "enqueue.hpp"
 
@@ -2865,22 +2866,14 @@ void axpy64(Ctx* ctx, const double* a, int64_t n, double s, double* x) {
 // Two launches an iteration (three on large systems). Every block sums the
 // partials of the launch before by itself, in the same fixed order, so alpha,
 // beta and the stopping test need no launch of one block of their own, and the
-// product forms its direction p = z + beta p as it gathers it. A scalar that one
-// launch reads and its block 0 also renews has a slot per parity of the
-// iteration. The host reads the state of a segment while the next one runs;
-// iterations after convergence return at once. The launches and the reads bound
-// it on small systems: with five launches an iteration and a read before each
-// next segment a mass solve of 31 k rows (32 iterations) took 907 us, now 731;
-// the leapfrog's, whose right-hand sides are on the device, 1,050 and 700 on
-// 111 k rows (36 iterations).
-struct CgS {
-  double rz[2];
-  long long iters[2];  // completed when the iteration of this parity starts
-  double bnorm2, rtol2, res2;
-  long long iter, max_iters;
-  int done;
-  int pad;
-};
+// product forms its direction p = z + beta p as it gathers it. What one launch
+// reads and its block 0 also renews, the stop among it, has a slot per parity of
+// the iteration (cg_state.hpp). The host reads the state of a segment while the
+// next one runs; iterations after convergence return at once. The launches and
+// the reads bound it on small systems: with five launches an iteration and a
+// read before each next segment a mass solve of 31 k rows (32 iterations) took
+// 907 us, now 731; the leapfrog's, whose right-hand sides are on the device,
+// 1,050 and 700 on 111 k rows (36 iterations).
 constexpr int CG_SEG = 8;  // even: a segment starts at parity 0
 constexpr int CG_RED = 1024, CG_ROWS = 2048;  // blocks at most: each block reads all partials
 // Rows up to which p is formed while gathered. Beyond, the two vectors miss the
@@ -2942,23 +2935,20 @@ __global__ void k_cg_start(CgS* S, const double* part, int np, double rtol, long
   double b = 0.0;
   for (int i = threadIdx.x; i < np; i += blockDim.x) b += part[CG_RR + i];
   const double bb = block_reduce(b, sh);
-  if (threadIdx.x == 0) {
-    CgS s{};
-    s.bnorm2 = bb;
-    s.rtol2 = rtol * rtol;
-    s.res2 = bb;
-    s.max_iters = max_iters;
-    s.done = (bb == 0.0 || max_iters <= 0) ? 1 : 0;
-    *S = s;
-  }
+  if (threadIdx.x == 0) *S = cg_first(bb, rtol, max_iters);
 }
 
+// First in the iteration's first launch: whether the run was over before it.
+__device__ __forceinline__ bool cg_begun_over(CgS* S, int par) {
+  if (!cg_stopped(*S, par)) return false;
+  if (blockIdx.x == 0 && threadIdx.x == 0) cg_put_stopped(*S, par);
+  return true;
+}
 // The scalars of the iteration's first launch: beta from the partials of r.z,
-// the stopping test on those of r.r (from the second iteration on; true: over).
+// the stopping test on those of r.r (true: over). Every thread of the block.
 __device__ __forceinline__ bool cg_begin(CgS* S, const double* part, int np, int par, double* sh,
                                          double& beta) {
-  const long long iter = S->iters[par], most = S->max_iters;
-  const double rz_old = S->rz[par], stop = S->rtol2 * S->bnorm2;
+  const CgRead q = cg_read(*S, par);  // not behind the barrier of the sums
   double rz = 0.0, rr = 0.0;
   for (int i = threadIdx.x; i < np; i += TPB) {
     rz += part[i];
@@ -2966,19 +2956,12 @@ __device__ __forceinline__ bool cg_begin(CgS* S, const double* part, int np, int
   }
   block_sums(rz, rr, sh);
   const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-  if (iter > 0 && (rr <= stop || iter >= most)) {
-    if (lead) {
-      S->res2 = rr;
-      S->iter = iter;
-      S->done = 1;
-    }
+  if (cg_stops(q, rr)) {
+    if (lead) cg_put_stop(*S, par, q, rr);
     return true;
   }
-  if (lead) {
-    S->rz[par ^ 1] = rz;
-    S->iters[par ^ 1] = iter + 1;
-  }
-  beta = iter > 0 ? rz / rz_old : 0.0;
+  if (lead) cg_put_next(*S, par, q, rz);
+  beta = cg_beta(q, rz);
   return false;
 }
 
@@ -3006,7 +2989,7 @@ __global__ void __launch_bounds__(TPB) k_cg_spmv(const int64_t* __restrict__ rp,
                                                  double* __restrict__ p1, double* __restrict__ ap,
                                                  CgS* S, double* part, int np, int par) {
   constexpr int U = SPMV_UNROLL;
-  if (S->done) return;
+  if (TWO ? cg_begun_over(S, par) : cg_over(*S, par)) return;
   __shared__ double sh[TPB / 64], sh2[TPB / 32];
   const int lane = threadIdx.x % LANES;
   const auto sums = [&](int64_t row, double& az, double& aq) {
@@ -3073,7 +3056,7 @@ __global__ void __launch_bounds__(TPB) k_cg_spmv(const int64_t* __restrict__ rp,
 __global__ void __launch_bounds__(TPB) k_cg_dir(const double* __restrict__ z, const double* __restrict__ p0,
                                                 double* __restrict__ p1, int64_t n, CgS* S, const double* part,
                                                 int np, int par) {
-  if (S->done) return;
+  if (cg_begun_over(S, par)) return;
   __shared__ double sh[TPB / 32];
   double beta = 0.0;
   if (cg_begin(S, part, np, par, sh, beta)) return;
@@ -3090,7 +3073,7 @@ __global__ void __launch_bounds__(TPB) k_cg_update(double* __restrict__ x, doubl
                                                    const double* __restrict__ ap,
                                                    const double* __restrict__ dinv, int64_t n,
                                                    const CgS* S, double* part, int np, int par) {
-  if (S->done) return;
+  if (cg_over(*S, par)) return;
   __shared__ double sh2[TPB / 32];
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   double xi = 0.0, pi = 0.0, ri = 0.0, ai = 0.0, di = 0.0;
@@ -3181,7 +3164,7 @@ KrylovStats cg_solve_ws(Ctx* ctx, const Csr& a, const double* dinv, const double
     if (seg == 0) continue;
     FEEC_HIP(hipEventSynchronize(ev[(seg - 1) & 1]));
     h = host[(seg - 1) & 1];
-    if (h.done) break;
+    if (cg_over(h, 1)) break;  // a segment ends on parity 1
   }
   // The segment in flight only returns, and its copy of the (final) state runs
   // before anything later on the stream reuses the state or the pinned words.

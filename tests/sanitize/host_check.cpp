@@ -1,7 +1,7 @@
 // Exercises the host-only code of libfeec (the meshers, option defaults,
 // status strings, element shapes, argument checks, the multigrid set-up's
-// dense Cholesky inverse and tridiagonal eigenvalue bisection, and the exact
-// (co)homology eliminations) in a build
+// dense Cholesky inverse and tridiagonal eigenvalue bisection, the exact
+// (co)homology eliminations, and the CG run's scalars) in a build
 // instrumented by AddressSanitizer and UndefinedBehaviorSanitizer. No GPU is
 // touched. Exit status 0 and the line "host_check ok" mean every check held.
 #include <cmath>
@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "feec.h"
+#include "../../formoniq_amd/csrc/cg_state.hpp"
 #include "../../formoniq_amd/csrc/feec_internal.hpp"
 
 static int failures = 0;
@@ -241,7 +242,47 @@ static void ingestion() {
   }
 }
 
+// The Jacobi CG's scalars, launch by launch: a wavefront that starts before the
+// lead thread has written and one that starts after decide alike, and once an
+// iteration has ended the run every later launch returns, whether it ended on
+// an even or an odd iteration, by residual or by budget.
+static void cg_scalars() {
+  using namespace feec;
+  const double rz = 3.0;
+  for (long long stop_at = 1; stop_at <= 9; ++stop_at)
+    for (int by_budget = 0; by_budget < 2; ++by_budget) {
+      CgS s = cg_first(4.0, 1e-3, by_budget ? stop_at : 1000);
+      EXPECT(!cg_over(s, 0) && !cg_over(s, 1));
+      long long ran = 0;
+      for (int it = 0; it < 24; ++it) {
+        const int par = it & 1;
+        const double rr = by_budget || it < stop_at ? 1.0 : 4e-6;
+        const CgS before = s;
+        const CgRead q = cg_read(before, par);
+        const bool over = cg_stopped(before, par), ends = !over && cg_stops(q, rr);
+        if (over)
+          cg_put_stopped(s, par);
+        else if (ends)
+          cg_put_stop(s, par, q, rr);
+        else
+          cg_put_next(s, par, q, rz + it);
+        const CgRead late = cg_read(s, par);
+        EXPECT(cg_stopped(s, par) == over);
+        EXPECT(cg_stops(late, rr) == cg_stops(q, rr));
+        EXPECT(cg_beta(late, rz + it) == cg_beta(q, rz + it));
+        EXPECT(cg_beta(q, rz + it) == (it == 0 ? 0.0 : (rz + it) / (rz + it - 1)) || it > stop_at);
+        EXPECT(cg_over(s, par) == (over || ends));
+        EXPECT(cg_over(s, par) == (it >= stop_at));
+        ran += !cg_over(s, par);
+      }
+      EXPECT(ran == stop_at && s.iter == stop_at && s.res2 == (by_budget ? 1.0 : 4e-6));
+    }
+  for (const CgS& none : {cg_first(0.0, 1e-3, 10), cg_first(1.0, 1e-3, 0)})
+    EXPECT(cg_stopped(none, 0) && cg_over(none, 0) && cg_over(none, 1) && none.iter == 0);
+}
+
 int main() {
+  cg_scalars();
   exact_topology();
   ingestion();
   meshers();

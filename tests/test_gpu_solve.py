@@ -594,3 +594,19 @@ def test_mass_cg_launch_forms(d, n, k):
         assert short.residual > 1e-11
     x0, zero = A.cg(0.0 * b, rtol=1e-11)
     assert zero.iters == 0 and zero.converged and not x0.any()
+
+
+@pytest.mark.parametrize("d,n,k", [(3, 9, 1), (3, 35, 1)])
+def test_mass_cg_budgets(d, n, k):
+    """CG runs ended by their budget on odd and even iterations, inside and at the
+    end of a host segment of 8, in both launch forms: the iterations reported are
+    the budget's, and each run's solution is the last one's next iterate (the
+    recurrence's residual, which only the finished iterations can have made,
+    equals the true one to 1e-12 of |b|)."""
+    _, _, gcx, geo, _, _ = both(d, n, 0.05, seed=n)
+    A = fa.WhitneyComplex(geo).mass(k)
+    b = np.cos(np.arange(A.shape[0]) * 0.9)
+    for most in (1, 2, 3, 7, 8, 9, 15, 16, 17):
+        x, rep = A.cg(b, rtol=1e-14, max_iters=most, raise_on_failure=False)
+        assert rep.iters == most and not rep.converged
+        assert abs(np.linalg.norm(A @ x - b) / np.linalg.norm(b) - rep.residual) <= 1e-12
