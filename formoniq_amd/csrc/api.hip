@@ -591,9 +591,10 @@ static int resolve_cheb_degree(const Problem& P) {
 // polynomial from the smallest grids on (assembly and solve, polynomial against
 // multigrid: 2D 16^2 k = 0 2.2 / 1.3 ms, 2D 32^2 k = 1 14.1 / 4.1, 3D 4^3 k = 1
 // 8.5 / 3.2, 3D 10^3 k = 2 23.9 / 8.1; requests from their mesh the same).
-// Below kMultigridAutoRows rows the polynomial stays where a caller chose its
-// degree, and for grade 2 of the relative complex, whose blocks need 70 to 80
-// iterations at every size (3D 6^3: 11.4 / 21.3 ms, 10^3: 21.6 / 21.9).
+// Below kMultigridAutoRows rows the polynomial stays where a caller set one of
+// its options (degree, interval, storage), and for grade 2 of the relative
+// complex, whose blocks need 70 to 80 iterations at every size (3D 6^3: 11.4 /
+// 21.3 ms, 10^3: 21.6 / 21.9).
 constexpr int64_t kMultigridAutoRows = 20000;
 // Chebyshev acceleration of the HX blocks: applications of B per block
 // application (cheb_degree = -1) and the interval's lower end as a fraction of
@@ -602,7 +603,8 @@ constexpr int kMultigridChebDefault = 5;
 constexpr double kMultigridChebFraction = 0.25;
 void problem_multigrid(Problem& P) {
   const int pc = P.opts.preconditioner;
-  const bool polynomial = P.opts.cheb_degree >= 0 || (P.k >= 2 && P.bc == FEEC_RELATIVE);
+  const bool polynomial = P.opts.cheb_degree >= 0 || P.opts.cheb_lower > 0.0 ||
+                          P.opts.precond_storage != FEEC_PC_STORE_SELL || (P.k >= 2 && P.bc == FEEC_RELATIVE);
   if (pc == FEEC_PC_CHEBYSHEV || (pc == FEEC_PC_AUTO && P.sys.n < kMultigridAutoRows && polynomial)) {
     P.sys.hx = nullptr;
     return;

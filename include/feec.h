@@ -112,7 +112,10 @@ typedef struct feec_solve_opts {
   double cheb_lower;     /* lower end of the Chebyshev interval as a fraction of its upper end
                             (1.05 lambda_max); 0 = by degree: 1e-2 up to degree 4, 3e-3 up to 8,
                             1.5e-3 up to 12, 1e-3 up to 32, 5e-4 up to 48, 2.5e-4 up to 64,
-                            1.2e-4 up to 96, else 6e-5 (default 0) */
+                            1.2e-4 up to 96, else 6e-5 (default 0). With the multigrid blocks,
+                            whose cheb_degree (default 5) is the applications of the auxiliary-
+                            space preconditioner per block, the lower end of their interval;
+                            0 = 1/4 */
   int32_t precond_storage; /* feec_pc_storage: how the matrix the polynomial runs on is
                               stored (default FEEC_PC_STORE_SELL) */
   int32_t preconditioner; /* feec_preconditioner: the block preconditioner (default FEEC_PC_AUTO) */
@@ -128,8 +131,9 @@ typedef struct feec_solve_opts {
  *   geometry from Euclidean coordinates and grade <= 2; otherwise FEEC_E_UNSUPPORTED.
  * FEEC_PC_CHEBYSHEV: a Chebyshev-Jacobi polynomial of degree cheb_degree on each block.
  * FEEC_PC_AUTO: multigrid where it applies, else Chebyshev; below 20,000 KKT rows also
- *   Chebyshev where cheb_degree >= 0 asks for a degree, and for grade 2 of the relative
- *   complex. Batched solves (feec_batch_run) always run Chebyshev. */
+ *   Chebyshev where one of the polynomial's options is set (cheb_degree >= 0,
+ *   cheb_lower > 0, precond_storage other than the default), and for grade 2 of the
+ *   relative complex. Batched solves (feec_batch_run) always run Chebyshev. */
 typedef enum {
   FEEC_PC_AUTO = 0,
   FEEC_PC_CHEBYSHEV = 1,

@@ -273,3 +273,27 @@ def test_auto_on_small_grids(d, n, k, rel):
         assert rep.converged and rep.residual <= 1e-10, rep.as_dict()
         u.append(np.concatenate(prob.solution()[:2]))
     assert np.linalg.norm(u[0] - u[1]) <= 1e-6 * np.linalg.norm(u[1])
+
+
+@pytest.mark.parametrize("opts,fmt", [(dict(cheb_lower=1e-2), "sell64_f16"), (dict(cheb_degree=12), "sell64_f16"),
+                                      (dict(precision=fa.FP64, precond_storage=fa.PC_CSR), "csr_f64"),
+                                      (dict(precision=fa.MIXED, precond_storage=fa.PC_CSR_HALF), "csr_f16"),
+                                      (dict(precision=fa.MIXED, precond_storage=fa.PC_CSR), "csr_f32")])
+def test_auto_keeps_the_polynomial_options(opts, fmt):
+    """Below 20,000 rows an option of the polynomial (degree, interval, storage)
+    means the polynomial to PC_AUTO: the same application as PC_CHEBYSHEV with it,
+    bit for bit. From there on, and with PC_MULTIGRID, the multigrid blocks run
+    whatever is set."""
+    _, _, gcx, geo, _, _ = both(3, 5, 0.05, seed=11)
+    wc = fa.WhitneyComplex(geo)
+    auto = fa.Problem(wc, 1, fa.solve_opts(**opts))
+    poly = fa.Problem(wc, 1, fa.solve_opts(preconditioner=fa.PC_CHEBYSHEV, **opts))
+    assert auto.preconditioner()["format"] == poly.preconditioner()["format"] == fmt
+    r = np.cos(np.arange(sum(auto.sizes)) * 0.4)
+    kind = dict(precision=opts.get("precision", fa.FP64_PC32), storage=opts.get("precond_storage", fa.PC_SELL))
+    np.testing.assert_array_equal(auto.apply_preconditioner(r, **kind), poly.apply_preconditioner(r, **kind))
+    multi = fa.Problem(wc, 1, fa.solve_opts(preconditioner=fa.PC_MULTIGRID, **opts))
+    assert multi.preconditioner()["format"].startswith("multigrid")
+    _, _, _, big, _, _ = both(2, 75, 0.05, seed=3)
+    large = fa.Problem(fa.WhitneyComplex(big), 1, fa.solve_opts(**opts))
+    assert sum(large.sizes) >= 20000 and large.preconditioner()["format"].startswith("multigrid")
