@@ -62,4 +62,13 @@ __host__ __device__ inline void cg_put_next(CgS& s, int par, const CgRead& q, do
 // iteration: whether the run is over.
 __host__ __device__ inline bool cg_over(const CgS& s, int par) { return s.stop[par ^ 1] != 0; }
 
+// Iterations of the host's segment `seg` (even: it starts at parity 0). The next
+// one is queued before a segment's state is read, so a run of one iteration (the
+// mass of the top grade is diagonal) waits for all launches of the first two. In
+// the form of three launches an iteration these are few: 384 k rows 513 us a
+// solve with eight and eight iterations in them, 448 with two and six. In the
+// form of two, sixteen iterations cost a short run less than the further read
+// costs the others (31 k rows, 29 iterations: 460 us and 472).
+constexpr int cg_segment(int seg, bool three) { return !three || seg > 1 ? 8 : seg == 0 ? 2 : 6; }
+
 }  // namespace feec

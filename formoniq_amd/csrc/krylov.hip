@@ -2874,7 +2874,6 @@ void axpy64(Ctx* ctx, const double* a, int64_t n, double s, double* x) {
 // read before each next segment a mass solve of 31 k rows (32 iterations) took
 // 907 us, now 731; the leapfrog's, whose right-hand sides are on the device,
 // 1,050 and 700 on 111 k rows (36 iterations).
-constexpr int CG_SEG = 8;  // even: a segment starts at parity 0
 constexpr int CG_RED = 1024, CG_ROWS = 2048;  // blocks at most: each block reads all partials
 // Rows up to which p is formed while gathered. Beyond, the two vectors miss the
 // caches (795 k rows: 59 us a product against 39) and p takes a launch of its own.
@@ -3143,12 +3142,13 @@ KrylovStats cg_solve_ws(Ctx* ctx, const Csr& a, const double* dinv, const double
   k_cg_init<<<gr, TPB, 0, st>>>(b, dinv, n, x, w.r, w.z, w.p, w.part);
   k_cg_start<<<1, TPB, 0, st>>>(w.S, w.part, (int)gr, rtol, (long long)max_iters);
   CgS h{};
+  const bool three = n > CG_TWO_ROWS;
   for (int seg = 0;; ++seg) {
-    for (int it = 0; it < CG_SEG; ++it) {
+    for (int it = 0; it < cg_segment(seg, three); ++it) {
       const int par = it & 1;
       double* p0 = par ? w.q : w.p;
       double* p1 = par ? w.p : w.q;
-      if (n <= CG_TWO_ROWS) {
+      if (!three) {
         k_cg_spmv<true><<<gs, TPB, 0, st>>>(a.row_ptr.p, a.col.p, a.val.p, n, w.z, p0, p1, w.ap, w.S, w.part,
                                             (int)gr, par);
       } else {

@@ -277,6 +277,12 @@ static void cg_scalars() {
       }
       EXPECT(ran == stop_at && s.iter == stop_at && s.res2 == (by_budget ? 1.0 : 4e-6));
     }
+  // a run of one iteration returns behind no more launches than eight iterations
+  // of five launches, the form whose state was read before the next segment
+  for (int three = 0; three < 2; ++three) {
+    for (int seg = 0; seg < 4; ++seg) EXPECT(cg_segment(seg, three) > 0 && cg_segment(seg, three) % 2 == 0);
+    EXPECT((2 + three) * (cg_segment(0, three) + cg_segment(1, three)) <= 5 * 8);
+  }
   for (const CgS& none : {cg_first(0.0, 1e-3, 10), cg_first(1.0, 1e-3, 0)})
     EXPECT(cg_stopped(none, 0) && cg_over(none, 0) && cg_over(none, 1) && none.iter == 0);
 }
