@@ -500,6 +500,21 @@ def run_step(args):
                       "iters": int(r.iters), "residual": float(r.residual)}), flush=True)
 
 
+def pc_product(pc, rows):
+    """The FP32 product by the preconditioner matrix P as the library runs it, from
+    Problem.preconditioner(): (kernel, description, bytes it cannot do without)."""
+    nnz, cb = int(pc["nnz"]), int(pc["column_bytes"])
+    if cb == 0:
+        # an FP32 value per entry; per row its number and its list's number, x read
+        # and y written once; the lists themselves (shared by the rows) not counted
+        return ("k_pc_lists<float>", "64-row slices with shared column-offset lists, a lane per row",
+                nnz * 4 + 16 * rows + 8 * (rows // 64 + 1))
+    # int16 column offsets (or int32) and FP32 values per entry, 8-byte row
+    # pointers, x read and y written once per row
+    return ("k_pc_spmv32<%s,4,2>" % ("short" if cb == 2 else "int"), "compressed rows, 4 lanes per row",
+            nnz * (cb + 4) + 8 * (rows + 1) + 8 * rows)
+
+
 def timed_steps(ctx, prob, steps, label):
     """Time `steps` steps (assemble + solve) of a resident problem."""
     lat, reps = [], []
@@ -642,18 +657,15 @@ def main():
         if tr.get("n_kkt") != n_kkt:
             tr = {}
     if mg is not None:
-        # an FP32 value per entry; per row its number and its list's number, x read
-        # and y written once; the lists themselves (shared by the rows) not counted
         p_rows, p_nnz = n_kkt, int(pc["nnz"])
-        spmv_bytes = p_nnz * 4 + 16 * p_rows + 8 * (p_rows // 64 + 1)
+        spmv_name, spmv_form, spmv_bytes = pc_product(pc, p_rows)
         achieved = spmv_bytes / mg["pc_spmv32"] / 1e9
         roof = {
-            "kernel": "k_pc_lists<float> (y = P x, the block-diagonal preconditioner matrix in FP32, "
-                      "64-row slices with shared column-offset lists, a lane per row)",
+            "kernel": f"{spmv_name} (y = P x, the block-diagonal preconditioner matrix in FP32, {spmv_form})",
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": tr.get("pc_spmv32_hbm_bytes_per_launch"),
             "algorithmic_bytes_per_launch": spmv_bytes, "launch_seconds": mg["pc_spmv32"],
-            "rows": p_rows, "nnz": p_nnz,
+            "rows": p_rows, "nnz": p_nnz, "column_bytes": int(pc["column_bytes"]),
         }
         nb0 = (args.n + 1) ** 3
         nv = 5  # slots of one 3D k = 1 cycle: sigma's V, u's gradient V and its 3 vector copies

@@ -841,9 +841,10 @@ class Problem:
 
     def preconditioner(self):
         """The block preconditioner as built: nonzeros, Chebyshev degree, lambda_max
-        per block, bytes per stored CSR column index, the format a solve with this
-        problem's options applies, the entries that format stores (SELL padding
-        included) and the off-diagonal nonzeros."""
+        per block, bytes per stored column index (0: rows hold the number of a shared
+        list of offsets in their place), the format a solve with this problem's options
+        applies, the entries that format stores (SELL padding included) and the
+        off-diagonal nonzeros."""
         nnz, deg, lam, cb = C.c_int64(), C.c_int32(), np.zeros(2), C.c_int32()
         fmt, stored, offd = C.c_int32(), C.c_int64(), C.c_int64()
         check(load().feec_problem_preconditioner(self._h, C.byref(nnz), C.byref(deg),

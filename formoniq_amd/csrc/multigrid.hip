@@ -3450,7 +3450,7 @@ void hx_kernel_times(Hx& h, int reps, bool use_graph, double out[4]) {
 
 void hx_info(const Hx& h, int* cheb_m, double lam[2], int* column_bytes) {
   if (cheb_m) *cheb_m = h.cheb_m;
-  if (column_bytes) *column_bytes = h.P_narrow ? 2 : 4;
+  if (column_bytes) *column_bytes = h.lists.on ? 0 : h.P_narrow ? 2 : 4;
   if (lam) {
     lam[0] = h.lam[0];
     lam[1] = h.lam[1];

@@ -453,8 +453,9 @@ typedef enum {
  * its nonzeros, the Chebyshev degree in use (0 = Jacobi; with the multigrid
  * preconditioner, the B applications per block application), the estimated
  * largest eigenvalue of D^-1 hdif_gram (with the multigrid preconditioner, of
- * B hdif_gram) per block, the bytes per stored CSR
- * column index (2 when every |col - row| fits a 16-bit offset, else 4), the
+ * B hdif_gram) per block, the bytes per stored
+ * column index (2 when every |col - row| fits a 16-bit offset, else 4; 0 where
+ * the rows hold the number of a shared list of offsets in their place), the
  * format a solve with the problem's options applies (feec_pc_format), the
  * entries that format stores (with SELL padding) and the off-diagonal
  * nonzeros; any pointer may be NULL. */

@@ -11,6 +11,7 @@ import pytest
 import scipy.sparse.linalg as spla
 
 import formoniq_amd as fa
+from bench import pc_product
 from oracle import oracle as o
 
 from _common import both
@@ -297,3 +298,17 @@ def test_auto_keeps_the_polynomial_options(opts, fmt):
     _, _, _, big, _, _ = both(2, 75, 0.05, seed=3)
     large = fa.Problem(fa.WhitneyComplex(big), 1, fa.solve_opts(**opts))
     assert sum(large.sizes) >= 20000 and large.preconditioner()["format"].startswith("multigrid")
+
+
+@pytest.mark.parametrize("n,column_bytes", [(60, 2), (384, 2), (400, 0)])
+def test_preconditioner_reports_its_rows(n, column_bytes):
+    """preconditioner()["column_bytes"] tells rows of columns from rows that hold a
+    list's number (from 150,000 rows on), and the benchmark's model of the product
+    by P follows it: the kernel's name, and per entry its value and its column."""
+    _, _, _, geo, _, _ = both(2, n, 0.05, seed=n)
+    prob = fa.Problem(fa.WhitneyComplex(geo, relative=True), 0, mg_opts())
+    pc, rows = prob.preconditioner(), sum(prob.sizes)
+    assert pc["column_bytes"] == column_bytes
+    name, _, nbytes = pc_product(pc, rows)
+    assert name.startswith("k_pc_spmv32" if column_bytes else "k_pc_lists")
+    assert 0 < nbytes - (4 + column_bytes) * pc["nnz"] <= 17 * rows + 16
