@@ -59,6 +59,7 @@
 // symmetric operator.
 #include <algorithm>
 #include <cmath>
+#include <limits>
 #include <map>
 #include <mutex>
 #include <string>
@@ -2434,19 +2435,32 @@ void bind_pc_matrix(Hx& h, const KktSystem& s) {
   FEEC_HIP(hipGetLastError());
 }
 
-// P's slices (k_pc_lists), where its rows repeat few enough offset lists and
-// there are enough of them that one lane a row fills the chip. FP32, us a product
-// in slices / as compressed rows, 3D k = 1: 118 k rows 7.7 / 7.0, 185 k 9.8 / 10.5,
-// 301 k 13.4 / 14.3, 531 k 18.2 / 20.3; 3D k = 2: 146 k 12.0 / 9.5, 363 k 14.8 /
-// 14.4 with the application 410.7 / 413.9; 2D k = 1: 136 k 6.3 / 6.8, 642 k 11.0 /
-// 14.2. Building the slices adds 0.2-0.4 ms to a 3D set-up (64^3: 37.0 -> 37.4).
-constexpr int64_t kListRows = 150000;
+// Rows from which P is kept in slices (k_pc_lists): one lane a row has to fill
+// the chip, and the entries saved have to outlast the set-up that finds the lists
+// (0.2 to 0.5 ms in 3D). FP32, us a product in slices / as compressed rows:
+//   2D k = 0  122 k rows 6.3 / 6.7, 202 k 6.8 / 7.7, 998 k 12.4 / 20.6
+//   2D k = 1  145 k 6.4 / 7.1, 293 k 7.5 / 9.6, 1.44 M 15.6 / 26.8
+//   3D k = 0  104 k 6.8 / 6.6, 141 k 7.8 / 9.0, 493 k 11.0 / 17.8
+//   3D k = 1  133 k 8.8 / 7.7, 205 k 10.9 / 11.0, 250 k 12.3 / 12.2, 358 k 14.5 /
+//             15.1, 422 k 16.2 / 18.0, 659 k 20.2 / 23.9
+//   3D k = 2  158 k 10.1 / 9.8, 344 k 15.7 / 14.5, 385 k 14.4 / 14.7, 429 k 15.4 /
+//             18.7, 1.24 M 39.0 / 44.5
+//   4D k = 1  194 k 23.2 / 23.3, 391 k 42.5 / 39.6; 4D k = 2 484 k 51.9 / 54.9
+// (a whole solve, 3D k = 2: 0.98 of the other's speed at 158 k, 0.98 at 385 k,
+// 1.00 at 429 k, 1.03 at 476 k). In FP64 a solve is 1 to 5% faster from 150 k rows
+// on, but for grade 2 beyond 2D, whose gathers bound it: 2% slower from 158 k to
+// 1.76 M rows.
+int64_t list_rows(int d, int k, bool fp32) {
+  if (d >= 3 && k >= 2 && !fp32) return std::numeric_limits<int64_t>::max();
+  return d >= 3 && k >= 1 && fp32 ? 400000 : 150000;
+}
+// P's slices, where its rows repeat few enough offset lists.
 void build_lists(Hx& h, const KktSystem& s) {
   Ctx* ctx = h.ctx;
   hipStream_t st = ctx->stream;
   Hx::Lists& l = h.lists;
   const int64_t n = s.P.nrows, nnz = s.P.nnz;
-  if (n < kListRows || n >= ((int64_t)1 << 31) - SELL_WIN) return;
+  if (n < list_rows(h.d, h.k, h.spectrum_fp32) || n >= ((int64_t)1 << 31) - SELL_WIN) return;
   DBuf<unsigned long long> keys(ctx, kListSlots);
   DBuf<unsigned int> rep(ctx, kListSlots);
   DBuf<int32_t> id(ctx, kListSlots), slot(ctx, n), len(ctx, n);

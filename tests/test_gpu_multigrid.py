@@ -14,7 +14,7 @@ import formoniq_amd as fa
 from bench import pc_product
 from oracle import oracle as o
 
-from _common import both
+from _common import both, kuhn_mesh
 
 pytestmark = pytest.mark.gpu
 
@@ -312,3 +312,18 @@ def test_preconditioner_reports_its_rows(n, column_bytes):
     name, _, nbytes = pc_product(pc, rows)
     assert name.startswith("k_pc_spmv32" if column_bytes else "k_pc_lists")
     assert 0 < nbytes - (4 + column_bytes) * pc["nnz"] <= 17 * rows + 16
+
+
+@pytest.mark.parametrize("d,n,k,rel,precision,slices", [
+    (2, 388, 0, True, fa.FP64_PC32, False), (2, 389, 0, True, fa.FP64_PC32, True),
+    (3, 30, 1, False, fa.FP64_PC32, False), (3, 37, 1, False, fa.FP64_PC32, True),
+    (3, 30, 1, False, fa.FP64, True), (3, 26, 2, False, fa.FP64_PC32, False),
+    (3, 28, 2, False, fa.MIXED, True), (3, 28, 2, False, fa.FP64, False), (2, 200, 2, False, fa.FP64, True)])
+def test_which_systems_take_slices(d, n, k, rel, precision, slices):
+    """P is kept in slices only where a solve gains by them: from 150,000 rows on,
+    in FP32 for grades 1 and 2 beyond 2D from 400,000 on, and in FP64 not for
+    grade 2 beyond 2D."""
+    cells, coords = kuhn_mesh(d, n, 0.05, seed=n)
+    geo = fa.MeshLengthsSq.from_coords(fa.Complex(d, cells, nverts=len(coords)), coords)
+    prob = fa.Problem(fa.WhitneyComplex(geo, relative=rel), k, mg_opts(precision=precision))
+    assert (prob.preconditioner()["column_bytes"] == 0) == slices, sum(prob.sizes)
