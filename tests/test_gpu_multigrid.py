@@ -24,7 +24,8 @@ def mg_opts(**kw):
 
 
 CASES = [(2, 12, 0.1, 1, False), (2, 13, 0.1, 1, True), (2, 10, 0.1, 0, False), (2, 9, 0.1, 2, True),
-         (3, 6, 0.05, 1, False), (3, 5, 0.05, 1, True), (3, 5, 0.05, 2, False), (3, 6, 0.05, 0, True)]
+         (3, 6, 0.05, 1, False), (3, 5, 0.05, 1, True), (3, 5, 0.05, 2, False), (3, 6, 0.05, 0, True),
+         (4, 2, 0.05, 2, False), (4, 3, 0.05, 2, True), (4, 3, 0.05, 1, True)]
 
 
 @pytest.mark.parametrize("m", [1, 4])
@@ -77,19 +78,21 @@ def test_hx_application_matches_oracle(d, n, amp, k, rel, m):
     assert np.abs(got_pc32 - want32).max() <= tol32 * scale
 
 
-@pytest.mark.parametrize("d,n,k,rel", [(2, 400, 0, True), (2, 200, 1, False), (3, 30, 1, True)])
+@pytest.mark.parametrize("d,n,k,rel", [(2, 400, 0, True), (2, 200, 1, False), (3, 30, 1, True), (3, 37, 1, False)])
 def test_chebyshev_products_on_lists(d, n, k, rel):
-    """From 150,000 rows on the Chebyshev steps multiply by P's slices with shared
-    offset lists (rows sorted by length in windows of 256, so the last window and
-    the slices of mixed lengths are ragged: the row counts are no multiples of 64).
-    One step (m = 2) against the oracle, in the problem's own precision (slices)
-    and in the other one (compressed rows). The nodal blocks (sigma, and u for
+    """The Chebyshev steps of large systems multiply by P's slices with shared offset
+    lists (rows sorted by length in windows of 256, so the last window and the
+    slices of mixed lengths are ragged: the row counts are no multiples of 64).
+    One step (m = 2) against the oracle, in the problem's own precision (slices;
+    for 3D 30^3 in FP32 still compressed rows) and in the other one (compressed
+    rows). The nodal blocks (sigma, and u for
     k = 0) to 1e-10 and 1e-4. For k = 1 the second step applies B to the rounding
     of P d, at most eps x 16 terms of a row, and B's nodal part carries rounding
     that P's own range lacks over with up to 1 / lambda_min = O(n^2) of itself:
-    16 eps n^2, eps 2^-53 and 2^-24 (1.9e-2 measured at n = 184 in FP32, 3.2e-2
-    bounded there; a wrong entry leaves errors of order one, and the same kernel holds
-    1e-10 in FP64)."""
+    16 eps n^2, eps 2^-53 and 2^-24. In FP32 that is 3.8e-2 in 2D (1.5e-2 measured),
+    too wide for a wrong value here and there, and 1.3e-3 in 3D at n = 37 (9.3e-4
+    measured); a wrong entry leaves errors of order one, and the same kernel holds
+    1e-10 in FP64."""
     ocx, oL, gcx, geo, _, coords = both(d, n, 0.05, seed=n)
     gc = fa.WhitneyComplex(geo, relative=rel)
     oc = o.WhitneyComplex(ocx, oL, relative=rel)
@@ -100,6 +103,7 @@ def test_chebyshev_products_on_lists(d, n, k, rel):
         prob.assemble()
         ns, nu, nh = prob.sizes
         assert ns + nu >= 150000 and (ns + nu) % 64
+        assert (prob.preconditioner()["column_bytes"] == 0) == (own == fa.FP64 or (d, n) != (3, 30))
         if r is None:
             r = np.sin(np.arange(ns + nu + nh) * 0.7 + 0.3)
         lam = prob.preconditioner()["lambda_max"]
@@ -245,6 +249,7 @@ def test_c2_full_size_multigrid():
 @pytest.mark.parametrize("d,n,k,rel", [(1, 9, 0, True), (2, 2, 1, False), (2, 3, 0, True), (2, 7, 0, False),
                                        (2, 16, 1, True), (2, 9, 2, False), (2, 8, 2, True), (3, 2, 1, False),
                                        (3, 5, 0, True), (3, 4, 2, False), (3, 4, 2, True), (4, 2, 1, False),
+                                       (4, 2, 2, False), (4, 3, 2, True),
                                        (4, 3, 0, True), (3, 3, 3, False)])
 def test_auto_on_small_grids(d, n, k, rel):
     """PC_AUTO on systems below 20,000 rows: multigrid wherever PC_MULTIGRID can be

@@ -65,11 +65,12 @@ def test_kkt_parity(d, n, amp, rel):
 @pytest.mark.parametrize("precision", [fa.FP64, fa.MIXED, fa.FP64_PC32])
 @pytest.mark.parametrize("d,n,amp", [(1, 16, 0.2), (2, 8, 0.1), (3, 4, 0.05)])
 @pytest.mark.parametrize("rel", [False, True])
-def test_solve_source(d, n, amp, rel, precision):
+@pytest.mark.parametrize("preconditioner", [fa.PC_AUTO, fa.PC_CHEBYSHEV])
+def test_solve_source(d, n, amp, rel, precision, preconditioner):
     ocx, oL, gcx, geo, _, _ = both(d, n, amp, seed=7)
     oc = o.WhitneyComplex(ocx, oL, relative=rel)
     gc = fa.WhitneyComplex(geo, relative=rel)
-    opts = fa.solve_opts(precision=precision)
+    opts = fa.solve_opts(precision=precision, preconditioner=preconditioner)
     for k in range(d + 1):
         f = fa.normal_vector(ocx.nsimplices(k), 1 + k)
         sig, u, p, rep = fa.solve_source(gc, f, k, opts)
@@ -135,10 +136,12 @@ def test_preconditioner_storage_variants_agree(precision):
     _, _, gcx, geo, _, _ = both(3, 5, 0.05, seed=11)
     gc = fa.WhitneyComplex(geo)
     f = fa.normal_vector(gcx.nsimplices(1), 12)
-    _, u64, _, r64 = fa.solve_source(gc, f, 1, fa.solve_opts(precision=fa.FP64, precond_storage=fa.PC_CSR))
+    _, u64, _, r64 = fa.solve_source(gc, f, 1, fa.solve_opts(precision=fa.FP64, precond_storage=fa.PC_CSR,
+                                                            preconditioner=fa.PC_CHEBYSHEV))
     assert r64.residual <= 1e-10
     for store in (fa.PC_SELL, fa.PC_CSR_HALF, fa.PC_CSR):
-        _, u, _, rep = fa.solve_source(gc, f, 1, fa.solve_opts(precision=precision, precond_storage=store))
+        _, u, _, rep = fa.solve_source(gc, f, 1, fa.solve_opts(precision=precision, precond_storage=store,
+                                                                preconditioner=fa.PC_CHEBYSHEV))
         assert rep.residual <= 1e-10, (store, rep.residual)
         assert np.linalg.norm(u - u64) <= 1e-8 * np.linalg.norm(u64), store
 
@@ -256,11 +259,13 @@ def test_fp64_pc32_solve():
     _, _, gcx, geo, _, _ = both(3, 6, 0.05, seed=13)
     gc = fa.WhitneyComplex(geo)
     f = fa.normal_vector(gcx.nsimplices(1), 14)
-    _, u64, _, r64 = fa.solve_source(gc, f, 1, fa.solve_opts(precision=fa.FP64))
-    _, u, _, rep = fa.solve_source(gc, f, 1, fa.solve_opts(precision=fa.FP64_PC32))
+    poly = dict(preconditioner=fa.PC_CHEBYSHEV)
+    _, u64, _, r64 = fa.solve_source(gc, f, 1, fa.solve_opts(precision=fa.FP64, **poly))
+    assert fa.Problem(gc, 1, fa.solve_opts(**poly)).preconditioner()["format"] == "sell64_f16"
+    _, u, _, rep = fa.solve_source(gc, f, 1, fa.solve_opts(precision=fa.FP64_PC32, **poly))
     assert rep.converged and rep.residual <= 1e-10, rep.as_dict()
     assert np.linalg.norm(u - u64) <= 1e-8 * np.linalg.norm(u64)
-    _, _, _, rmix = fa.solve_source(gc, f, 1, fa.solve_opts(precision=fa.MIXED))
+    _, _, _, rmix = fa.solve_source(gc, f, 1, fa.solve_opts(precision=fa.MIXED, **poly))
     assert rep.iters <= rmix.iters, (rep.as_dict(), rmix.as_dict())
     for store in (fa.PC_CSR_HALF, fa.PC_CSR):
         with pytest.raises(fa.FeecError):
@@ -280,10 +285,11 @@ def test_fp64_pc32_solve():
     assert np.linalg.norm(prob.solution()[1] - u64) <= 1e-8 * np.linalg.norm(u64)
 
 
-def test_resident_problem_reassembly_and_device_source():
+@pytest.mark.parametrize("preconditioner", [fa.PC_AUTO, fa.PC_CHEBYSHEV])
+def test_resident_problem_reassembly_and_device_source(preconditioner):
     _, _, gcx, geo, _, _ = both(3, 4, 0.05, seed=2)
     gc = fa.WhitneyComplex(geo)
-    prob = fa.Problem(gc, 1, fa.solve_opts(precision=fa.MIXED))
+    prob = fa.Problem(gc, 1, fa.solve_opts(precision=fa.MIXED, preconditioner=preconditioner))
     f = fa.normal_vector(gcx.nsimplices(1), 9)
     r1 = prob.solve(f)
     s1, u1, _ = prob.solution()
