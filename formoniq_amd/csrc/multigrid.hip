@@ -2014,23 +2014,30 @@ __global__ void k_gather_entries(const int64_t* seg, const uint32_t* src, const 
   out[q] = in[(int64_t)src[seg[e]] * C + (q - e * C)];
 }
 
-// (D Pi)'s values on the pattern of `rp`, `col` (which holds every column of the
-// product's row): entry (r, v) takes sum_q D(r, q) Pi(q, v), C values.
+// (D Pi)'s values on the pattern of `rp`, `col`: entry (r, v) takes
+// sum_q D(r, q) Pi(q, v), C values; bad[0] set when a column of the product's row
+// is not in the pattern's.
 __global__ void k_compose(const int64_t* rp, const int32_t* col, int64_t nrows, const int64_t* drp,
                           const int32_t* dcol, const double* dval, const int64_t* prp, const int32_t* pcol,
-                          const double* pval, int C, double* out) {
+                          const double* pval, int C, double* out, int* bad) {
   const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (r >= nrows) return;
+  int64_t left = 0;  // terms without a place
+  for (int64_t q = drp[r]; q < drp[r + 1]; ++q) left += prp[dcol[q] + 1] - prp[dcol[q]];
   for (int64_t p = rp[r]; p < rp[r + 1]; ++p)
     for (int v = 0; v < C; ++v) {
       double acc = 0.0;
       for (int64_t q = drp[r]; q < drp[r + 1]; ++q) {
         const int32_t e = dcol[q];
         for (int64_t s = prp[e]; s < prp[e + 1]; ++s)
-          if (pcol[s] == col[p]) acc += dval[q] * pval[s * C + v];
+          if (pcol[s] == col[p]) {
+            acc += dval[q] * pval[s * C + v];
+            left -= v == 0;
+          }
       }
       out[p * C + v] = acc;
     }
+  if (left) atomicOr(bad, 1);
 }
 
 // [a | b] on one pattern: a's C_a values, then b's C_b values, per entry;
@@ -2201,8 +2208,8 @@ void interleave_dev(Ctx* ctx, const XCsr& a, const XCsr& b, XCsr& out, int* bad)
   finish_x(ctx, out);
 }
 
-// D Pi on the pattern of `like` (which covers the product's).
-void compose_dev(Ctx* ctx, const XCsr& D, const XCsr& Pi, const XCsr& like, XCsr& out) {
+// D Pi on the pattern of `like`; bad: that does not cover the product's.
+void compose_dev(Ctx* ctx, const XCsr& D, const XCsr& Pi, const XCsr& like, XCsr& out, int* bad) {
   const Csr& lm = like.m;
   Csr& c = out.m;
   c.ctx = ctx;
@@ -2218,7 +2225,7 @@ void compose_dev(Ctx* ctx, const XCsr& D, const XCsr& Pi, const XCsr& like, XCsr
     FEEC_HIP(hipMemcpyAsync(c.col.p, lm.col.p, lm.nnz * 4, hipMemcpyDeviceToDevice, ctx->stream));
     k_compose<<<grid_for(lm.nrows), TPB, 0, ctx->stream>>>(lm.row_ptr.p, lm.col.p, lm.nrows, D.m.row_ptr.p,
                                                            D.m.col.p, D.m.val.p, Pi.m.row_ptr.p, Pi.m.col.p,
-                                                           Pi.m.val.p, out.C, c.val.p);
+                                                           Pi.m.val.p, out.C, c.val.p, bad);
   }
   FEEC_HIP(hipGetLastError());
   finish_x(ctx, out);
@@ -2773,10 +2780,13 @@ Hx* hx_create(Geom& g, int bc, int k, const KktSystem& s, int sweeps, int cheb_m
       vector_nodal_dev(m, X, 1, order_l.p, live_col_dev, nl, nb0, Pl);
       // the curl part's copies enter and leave through D_1 Pi_1, on Pi_2's pattern
       // (a face's live vertices hold those of its edges)
-      compose_dev(ctx, b.o_d, Pl, Pi, DPl);
       DBuf<int> bad(ctx, 1);
       k_zero_i32<<<1, 64, 0, ctx->stream>>>(bad.p, 1);
+      compose_dev(ctx, b.o_d, Pl, Pi, DPl, bad.p);
       interleave_dev(ctx, Pi, DPl, b.o_main, bad.p);
+      int hb = 0;
+      copy_to_host(ctx, &hb, bad.p, sizeof(hb));
+      FEEC_REQUIRE(hb == 0, FEEC_E_DEVICE, "transfer patterns differ");
       transpose_dev(ctx, b.o_d, b.g_t);
       transpose_dev(ctx, b.o_main, b.g_main);
       b.slot_main = slot;
