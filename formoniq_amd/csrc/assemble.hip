@@ -236,6 +236,10 @@ __global__ void k_diag(const int64_t* row_ptr, const int32_t* col, const double*
 
 }  // namespace
 
+void require_entries(int64_t total) {
+  FEEC_REQUIRE(total < (int64_t(1) << 31), FEEC_E_ARG, "too many contributions for one matrix");
+}
+
 void coo_plan_build(Ctx* ctx, CooPlan& plan, int64_t nrows, int64_t ncols, int64_t n,
                     const int32_t* rows, const int32_t* cols, const uint32_t* srcs) {
   plan.nrows = nrows;
@@ -277,7 +281,7 @@ void coo_plan_build(Ctx* ctx, CooPlan& plan, int64_t nrows, int64_t ncols, int64
   FEEC_HIP(hipMemcpyAsync(&hv, nvalid.p, sizeof(hv), hipMemcpyDeviceToHost, ctx->stream));
   ctx->sync();
   int64_t nv = (int64_t)hv;
-  FEEC_REQUIRE(nv < (int64_t(1) << 31), FEEC_E_ARG, "too many contributions for one matrix");
+  require_entries(nv);
   DBuf<int32_t> head(ctx, std::max<int64_t>(nv, 1)), scan(ctx, std::max<int64_t>(nv, 1));
   int64_t nnz = 0;
   if (nv > 0) {
@@ -688,6 +692,7 @@ void csr_block(Ctx* ctx, int nb, const BlockRef* blocks, const int64_t* row_size
       total += blocks[i].a->nnz;
       transposed = transposed || (blocks[i].transpose && blocks[i].a->nnz);
     }
+  require_entries(total);
   if (!transposed) {
     // the blocks' rows side by side: sorted already, no entry twice
     const int64_t n = roff[nb];
@@ -759,6 +764,7 @@ void csr_add(const Csr& a, const Csr& b, Csr& out) {
   Ctx* ctx = a.ctx;
   const int64_t n = a.nrows;
   FEEC_REQUIRE(n == b.nrows && a.ncols == b.ncols, FEEC_E_ARG, "csr_add shape mismatch");
+  require_entries(a.nnz + b.nnz);
   out.ctx = ctx;
   out.nrows = n;
   out.ncols = a.ncols;

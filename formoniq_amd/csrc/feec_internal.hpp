@@ -176,6 +176,10 @@ void release_cache(Ctx* ctx);
 void copy_to_device(Ctx* c, void* dst, const void* src, size_t bytes);
 void copy_to_host(Ctx* c, void* dst, const void* src, size_t bytes);
 
+// Refuses a matrix built from 2^31 contributions or more: plans count them in
+// 32 bits, and every way to build one refuses the same.
+void require_entries(int64_t total);
+
 // Device COO -> CSR plan: the sorted order of (row, col) keys, kept so that a
 // later value pass is a segmented sum (duplicates summed in input order).
 // A COO source index with this bit set contributes its value negated.

@@ -287,8 +287,14 @@ static void cg_scalars() {
     EXPECT(cg_stopped(none, 0) && cg_over(none, 0) && cg_over(none, 1) && none.iter == 0);
 }
 
+static void entry_limit() {
+  for (int64_t total : {int64_t(0), int64_t(1), (int64_t(1) << 31) - 1, int64_t(1) << 31, int64_t(1) << 33})
+    EXPECT((feec::guard([&] { feec::require_entries(total); }) == FEEC_OK) == (total < (int64_t(1) << 31)));
+}
+
 int main() {
   cg_scalars();
+  entry_limit();
   exact_topology();
   ingestion();
   meshers();
