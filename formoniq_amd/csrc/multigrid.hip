@@ -312,11 +312,12 @@ __host__ __device__ constexpr int tail_offset(int m) {
 // correction and two sweeps. A workgroup takes one slot of a tile and
 // recomputes the halo, its vectors in LDS, its vertices' operator rows in
 // registers: one launch in place of three. A lone workgroup takes about 6 us
-// (4 of them its loads), so this pays where all of them run at once, on levels
-// whose separate kernels are bound by the launch: 3D 21^3, 5 slots: 16 us
-// against 26 for the six, 17^3: 15 against 22; with more workgroups than the
-// chip holds the halo's work costs more than the launches (65^3: 75 against
-// 50, 28^3 with 10 slots: 31 against 28).
+// (4 of them its loads). In 3D this pays where all of them run at once, on levels
+// whose separate kernels are bound by the launch (21^3, 5 slots: 16 us against 26
+// for the six, 17^3: 15 against 22); with more workgroups than CUs the halo's
+// work costs more than the launches (65^3: 75 against 50, 28^3 with 10 slots: 31
+// against 28). In 2D a tile's halo is a fifth of it and the one read of the
+// operator in place of three decides at every size (LevelTiles::use).
 constexpr int TILE_TPB = 512;
 template <int D>
 constexpr int kTile = D == 1 ? 128 : D == 2 ? 16 : 4;  // coarse vertices an axis of a tile
@@ -2836,6 +2837,9 @@ Hx* hx_create(Geom& g, int bc, int k, const KktSystem& s, int sweeps, int cheb_m
     const int64_t nbv = (int64_t)l.box.nb * h->nv;
     if (i + 1 < h->L.size()) {
       bytes += (int64_t)(2 * h->sweeps) * ((int64_t)(NS / 2 + 1) * l.box.nb * 4 + 12 * nbv) + 16 * nbv;
+      // a level in two launches counts as its separate kernels too: with two
+      // the segments grow, and the graph built by a first solve with them (3D 16^3
+      // 3141 -> 3366 us) without a gain for the next ones
       if (i < h->tail32) launches += 2 + 2 * h->sweeps;
     } else {
       bytes += (int64_t)l.box.nb * l.box.nb * 4;
@@ -3023,11 +3027,15 @@ struct LevelTiles {
     down = cpow(nd, d);
     up = cpow(nu, d);
   }
-  // whether the level takes k_st_down / k_st_up: two sweeps, and no more
-  // workgroups than run at once (two a CU in 3D; 2D's use fewer registers and
-  // recompute less). On one side 21^3, 5 slots: 16 us against 26 in separate
-  // launches; on the other 65^3: 75 against 50.
-  bool use(const Hx& h) const { return d <= 3 && h.sweeps == 2 && std::max(down, up) * h.nv <= (d == 3 ? 512 : 2048); }
+  // Whether the level takes k_st_down / k_st_up: two sweeps, and in 3D, where the
+  // halo costs as much as the tile, no more workgroups than CUs, whose launches
+  // then bound the separate kernels. An application's time without tiles / with
+  // them on every level, us: 3D with 135 workgroups on the finest level (20^3,
+  // k = 1) 35.4 / 34.2, 216 (40^3, k = 0) 47.7 / 46.0; 270 (16^3, k = 2) 35.7 /
+  // 38.7, 320 (24^3, k = 1) 44.5 / 46.0, 343 (48^3, k = 0) 53.0 / 55.5, 625 (32^3,
+  // k = 1) 53.7 / 65.2. In 1D and 2D the tiles win at every size: 2D 300^2 k = 0
+  // 52.9 / 41.9, 1000^2 k = 1 291.8 / 225.0, 2400^2 k = 0 360.4 / 259.7.
+  bool use(const Hx& h) const { return d <= 3 && h.sweeps == 2 && (d < 3 || std::max(down, up) * h.nv <= 256); }
 };
 
 // The grid of the plain level kernels: vertices by slots.

@@ -12,13 +12,15 @@ from _common import both
 
 pytestmark = pytest.mark.gpu
 
-# (d, n, k, relative, sweeps): two-launch levels from 13^3 and 46^2 vertices on, partial last
+# (d, n, k, relative, sweeps): two-launch levels from 13^3 and 46^2 vertices on (in 3D
+# up to 256 workgroups: 16^3 with 10 slots and 24^3 with 5 have more), partial last
 # tiles, odd grids whose coarse box overhangs, a whole cycle in one launch (the largest and
 # one smaller; 1D below, at and beyond the 2,048 vertices of one workgroup), 4D (no tiles), one
 # and three sweeps (no tiles; the iterates change buffers)
 CASES = [(1, 300, 0, True, 2), (1, 900, 0, True, 2), (1, 2046, 0, True, 2), (1, 2047, 0, True, 2),
          (1, 2048, 0, True, 2), (1, 5000, 0, True, 2), (2, 44, 1, False, 2), (2, 45, 1, True, 2), (2, 66, 0, True, 2),
          (2, 97, 1, False, 2), (3, 11, 1, False, 2), (3, 12, 1, True, 2), (3, 13, 2, True, 2), (3, 15, 1, False, 2),
+         (3, 16, 2, False, 2), (3, 24, 1, False, 2),
          (3, 17, 0, True, 2), (3, 26, 0, True, 2), (4, 4, 1, False, 2), (2, 50, 1, False, 3), (3, 12, 1, False, 1),
          (3, 13, 1, True, 3)]
 
