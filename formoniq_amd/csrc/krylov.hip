@@ -2877,7 +2877,11 @@ void axpy64(Ctx* ctx, const double* a, int64_t n, double s, double* x) {
 constexpr int CG_RED = 1024, CG_ROWS = 2048;  // blocks at most: each block reads all partials
 // Rows up to which p is formed while gathered. Beyond, the two vectors miss the
 // caches (795 k rows: 59 us a product against 39) and p takes a launch of its own.
-constexpr int64_t CG_TWO_ROWS = 300000;
+// A solve in two / three launches an iteration, us, edges of 3D grids: 31 k rows
+// 525 / 523, 161 k 980 / 989, 197 k 1138 / 1118, 239 k 1213 / 1167, 286 k 1388 /
+// 1312, 463 k 1892 / 1734, 795 k 2815 / 2529; 3D faces 169 k 774 / 806, 329 k 1171
+// / 1119; 2D edges 30 k 569 / 598, 271 k 872 / 868, 481 k 1168 / 1126.
+constexpr int64_t CG_TWO_ROWS = 200000;
 constexpr int CG_RR = CG_RED, CG_PAP = 2 * CG_RED;  // places of the partials
 static_assert(CG_PAP + CG_ROWS <= 2 * NBLK, "CG partials fit their area");
 

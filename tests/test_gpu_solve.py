@@ -581,7 +581,7 @@ def test_harmonics_outside_a_ball(shape):
 @pytest.mark.parametrize("d,n,k", [(1, 3, 0), (2, 5, 1), (2, 63, 0), (3, 9, 3), (3, 24, 1), (3, 35, 1)])
 def test_mass_cg_launch_forms(d, n, k):
     """Jacobi CG on mass matrices from a few rows (one block, fewer rows than a
-    block's share) to beyond the two-launch form's 300,000 (3D 35^3 edges: 309 k):
+    block's share) to beyond the two-launch form's 200,000 (3D 35^3 edges: 309 k):
     the solution satisfies the system to the stop's rtol (the recurrence's
     residual follows the true one to roundoff, 1e-14 of |b| per iteration), a
     budget that ends the run is reported as such, and a zero right-hand side
