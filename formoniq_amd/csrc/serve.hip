@@ -12,7 +12,7 @@
 // upload sources, and the MINRES runs of all requests advance in lockstep, one
 // launch per phase covering every request that is still running (each with
 // the blocks and partial sums of a solve on its own, so results equal single
-// solves bit for bit).
+// solves with the same preconditioner, the polynomial, bit for bit).
 //
 // Server: `max_inflight` slots, each a worker thread with its own stream. A
 // queued request is admitted when a slot is free and its estimated resident

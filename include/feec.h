@@ -535,7 +535,9 @@ typedef struct feec_result {
 /* Batched: all element matrices of all requests in one persistent launch over
  * a (mesh, cell-range) work queue, then the solves with their MINRES runs in
  * lockstep (one launch per phase for every request still running); results
- * equal single solves bit for bit. */
+ * equal single solves with the same preconditioner bit for bit. FEEC_PC_AUTO
+ * means FEEC_PC_CHEBYSHEV here, and to a single solve of a Kuhn grid mostly
+ * the multigrid blocks: those agree to the residual tolerance. */
 feec_status feec_batch_run(feec_ctx *ctx, int nreq, const feec_request *reqs,
                            const feec_solve_opts *opts, feec_result *results);
 
